@@ -183,6 +183,14 @@ struct MatmulArgs {
     float* xsum;
 };
 hipError_t launch_matmul(const MatmulArgs& a, hipStream_t stream);
+// The tile form, any weight type: the x pre-pass in tile order (xh: 2 x in_dim
+// halves for each row of the batch rounded up to 64; xexp: splits x batch
+// exponents; Q4_K xsum: 1024 floats for each 64 rows and super-block), the
+// product kernel, and with splits > 1 (split_out: splits x batch x out_dim) the
+// ordered sum of the ranges.  K-quant ranges are whole super-blocks
+// (chunks_per_split a multiple of 4); 32 weight rows stay below 2 GiB.
+hipError_t launch_matmul_tile(const MatmulArgs& a, hipStream_t stream);
+int matmul_tile_rows();  // weight rows per workgroup
 // The small-batch form (batch <= 64, Q8_0, Q4_K or Q6_K weights): the x pre-pass in
 // tile order (xh: matmul_small_x_halves halves, xexp: splits x batch
 // exponents, one per K range of each row; for Q4_K also xsum), then one

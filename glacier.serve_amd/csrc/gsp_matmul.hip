@@ -6,8 +6,9 @@
 // Q8_0 (blocks of 32 int8 with an fp16 scale d: w = d * q), or the K-quant
 // super-blocks Q4_K and Q6_K (256 weights each, decoded further down).
 //
-// Two forms.  The fp32 form (matmul_batch_kernel, every F32 product and the
-// quantized ones too small for the fp16 forms): every weight is exact in fp32
+// Three forms.  The tile form (matmul_tile_kernel, described further down) takes
+// every product with enough work.  The fp32 form (matmul_batch_kernel, smaller
+// F32 products and the quantized ones too small for the fp16 forms): every weight is exact in fp32
 // (Q8_0's d * q has at most 19 significant bits), and the products run on
 // v_mfma_f32_16x16x4f32 with fp32 accumulation, so no operand is rounded below
 // fp32.  The fp16 forms
@@ -1281,6 +1282,820 @@ __global__ __launch_bounds__(kMmThreads, 2) void matmul_q6k_f16_small_kernel(Mat
     small_finish<NT>(a, acc, mt, nt0, n, g, tid, last);
 }
 
+// ---- The tile form: products with enough work to fill the chip -----------------
+//
+// matmul_tile_kernel<WT>.  matmul_f16_kernel and matmul_batch_kernel expand (or
+// load) a weight for every 64 rows x 16 weight rows of a wave and read each x
+// operand for one matrix step; instruction issue and LDS, not the matrix cores,
+// bound them.  Here a workgroup owns 64 batch rows (four M tiles of 16) and 128
+// weight rows, wave w the two N tiles (32 weight rows) from 32 w: an x operand
+// staged in LDS serves all four waves and two N tiles, and a wave expands its
+// own rows' words to fp16 operands in registers once per chunk of 64 k and uses
+// each for four M tiles.  Measured at 1024 rows of 4096 x 4096 (us): Q8_0 177 ->
+// 113, Q4_K 185 -> 102, Q6_K 194 -> 136, F32 279 -> 166, about 700 TFLOP/s of
+// fp16 matrix steps; what is left is instruction issue (a chunk of Q6_K is
+// 48 matrix steps and 130 vector instructions a wave; dropping the expansion
+// or the scaling takes it to 128 us each, the barriers nothing).
+//
+// x comes from matmul_split_x_tile_kernel as scaled fp16 pairs in the order the
+// operands are read, so a chunk of the workgroup's 64 rows is 16 KB in one
+// piece and goes to LDS with direct loads, a ring of four chunks with one barrier each.
+//
+// The k order inside a chunk is free as long as both operands agree, so each
+// weight type takes the order in which a lane's words are contiguous (KOrder):
+//   Q8_0: chunk c, block blk, lane group g: k = 64 c + 32 blk + 8 g ..; the
+//     block's int8 values are exact in fp16, its sum goes to a fresh
+//     accumulator that its scale adds to the running one.
+//   Q4_K: lane group g owns quarter g of the super-block (sub-blocks 2 g and
+//     2 g + 1, 32 contiguous quant bytes).  sc * (q - 8) is exact in fp16, so
+//     only d remains outside, one fma per chunk.  The min term dmin m - 8 d sc
+//     is two matrix steps per super-block: the 8 sub-block sums of x as fp16
+//     pairs (from the pre-pass, times 2^-6) against the 6-bit mins and scales.
+//   Q6_K: lane group g owns l = 16 (g % 2) .. + 15 of each quarter of half
+//     g / 2.  m = sc * (q - 32), at most 4096, takes two halves: its fp16
+//     rounding and the rest (0 or +-1), three matrix steps instead of the four
+//     that scaling each 16 weights apart takes.
+//   F32: as Q8_0, but a lane's eight values are k = 32 blk + 4 g .. + 3 and 16
+//     further on, so that one load instruction covers 64 contiguous bytes of
+//     each row.  They enter as an fp16 pair scaled by the row's largest |w| of
+//     the chunk (2^e, applied with the chunk's sum); as for x, the pair keeps all
+//     but ~2^-24 of the element, and the lo x lo product (at most 2^-24,
+//     typically 2^-27 of the term) is left out.  Against float64 the products
+//     are closer than the fp32 form's (4096 x 4096 at 256 rows: 8.4e-7 ->
+//     1.5e-7): a running sum rounds once a chunk instead of once per four k.
+// K is split over ranges only where the tiles leave CUs idle; the ranges' sums
+// are then added in order by matmul_reduce_kernel.
+template <int WT>
+struct KOrder {
+    // Where the eight values from k (a multiple of 8) go: chunk, block and lane group
+    // (F32: see matmul_split_x_tile_kernel).
+    static __device__ __forceinline__ void place(int k, int& c, int& blk, int& g) {
+        if constexpr (WT == kWeightQ4_K) {
+            c = 4 * (k >> 8) + 2 * ((k >> 4) & 1) + ((k >> 5) & 1);
+            g = (k >> 6) & 3;
+            blk = (k >> 3) & 1;
+        } else if constexpr (WT == kWeightQ6_K) {
+            c = 4 * (k >> 8) + ((k >> 5) & 3);
+            g = 2 * ((k >> 7) & 1) + ((k >> 4) & 1);
+            blk = (k >> 3) & 1;
+        } else {
+            c = k >> 6;
+            blk = (k >> 5) & 1;
+            g = (k >> 3) & 3;
+        }
+    }
+};
+
+// Added to a row's exponent when the fp16 pairs cannot stand for the row (F32
+// products: an infinite element, or a row whose largest |x| is below 2^-113):
+// its outputs are summed in plain fp32 instead.
+constexpr int kXPlain = 1 << 16;
+constexpr int kTileHalves = 2048;   // one M tile of a chunk: [block][hi, lo][lane][8 halves]
+constexpr int kXBlockSumLog2 = 6;   // Q4_K's sub-block sums of x enter times 2^-6 (32 values below 2^13 each)
+
+// x of batch row b over K range z as scaled fp16 pairs in tile order,
+// [64-row group][chunk][M tile][block][hi, lo][lane g * 16 + m][8 halves], with
+// the exponent xexp[z][b]: as matmul_split_x_kernel, mx * 2^-e in [2^12, 2^13).
+template <int WT>
+__global__ __launch_bounds__(kMmThreads) void matmul_split_x_tile_kernel(MatmulArgs a) {
+    __shared__ float red[kMmThreads / 64];
+    const int b = blockIdx.x;
+    const int z = blockIdx.y;
+    const int t = threadIdx.x;
+    const int p0 = z * a.chunks_per_split * 8;  // pieces of eight values
+    const int np = min(a.in_dim / 8, p0 + a.chunks_per_split * 8) - p0;
+    const f4* xr = reinterpret_cast<const f4*>(a.x + (int64_t)b * a.in_dim) + 2 * (int64_t)p0;
+    // Ranges of up to 8192 values stay in registers between the two passes; longer ones are read twice.
+    constexpr int kHeld = 4;
+    const bool held = np <= kHeld * kMmThreads;
+    f4 hv[kHeld][2];
+    float mx = 0.f;
+    auto max8 = [&](const f4& u, const f4& v) {
+        const float mu = fmaxf(fmaxf(fabsf(u[0]), fabsf(u[1])), fmaxf(fabsf(u[2]), fabsf(u[3])));
+        const float mv = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+        mx = fmaxf(mx, fmaxf(mu, mv));
+    };
+    if (held) {
+#pragma unroll
+        for (int j = 0; j < kHeld; ++j)
+            if (kMmThreads * j < np) {
+                const int i = min(t + kMmThreads * j, np - 1);
+                hv[j][0] = xr[2 * i];
+                hv[j][1] = xr[2 * i + 1];
+            }
+#pragma unroll
+        for (int j = 0; j < kHeld; ++j)
+            if (kMmThreads * j < np) max8(hv[j][0], hv[j][1]);
+    } else {
+#pragma unroll 4
+        for (int i = t; i < np; i += kMmThreads) max8(xr[2 * i], xr[2 * i + 1]);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+    if ((t & 63) == 0) red[t >> 6] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    int ex = 0;
+    if (mx > 0.f && mx <= FLT_MAX) (void)frexpf(mx, &ex);
+    const int e = mx > 0.f ? (mx <= FLT_MAX ? min(115, max(-126, ex - 13)) : 115) : 0;
+    const float down = ldexpf(1.0f, -e);
+    _Float16* xt = static_cast<_Float16*>(a.xh);
+    const int64_t chunks = a.in_dim / 64;
+    const int64_t row0 = (int64_t)(b >> 6) * chunks;  // chunks before the row's group
+    const int tile = (b >> 4) & 3;
+    const int m = b & 15;
+    auto put = [&](int i, const f4& r0, const f4& r1) {
+        h8 hi, lo;
+        float sm = 0.f;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const float v = (q < 4 ? r0[q & 3] : r1[q & 3]) * down;
+            hi[q] = (_Float16)v;
+            // An infinite element rides on its hi half alone (Inf - Inf would be NaN).
+            lo[q] = (_Float16)(__builtin_isinf(v) ? 0.f : v - (float)hi[q]);
+            sm += v;
+        }
+        const int k = 8 * (p0 + i);
+        int c, blk, g;
+        KOrder<WT>::place(k, c, blk, g);
+        _Float16* dst = xt + ((row0 + c) * 4 + tile) * kTileHalves + blk * 1024;
+        if constexpr (WT == kWeightF32) {
+            // The two fours from k and k + 4 go to lane groups (k / 4) % 4 and the next, first or second half.
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                _Float16* d4 = dst + ((((k >> 2) + q) & 3) * 16 + m) * 8 + 4 * ((k >> 4) & 1);
+                *reinterpret_cast<h4v*>(d4) = q ? __builtin_shufflevector(hi, hi, 4, 5, 6, 7) : __builtin_shufflevector(hi, hi, 0, 1, 2, 3);
+                *reinterpret_cast<h4v*>(d4 + 512) = q ? __builtin_shufflevector(lo, lo, 4, 5, 6, 7) : __builtin_shufflevector(lo, lo, 0, 1, 2, 3);
+            }
+        } else {
+            *reinterpret_cast<h8*>(dst + (g * 16 + m) * 8) = hi;
+            *reinterpret_cast<h8*>(dst + (g * 16 + m) * 8 + 512) = lo;
+        }
+        if constexpr (WT == kWeightQ4_K) {
+            // Four consecutive threads hold a sub-block's 32 values.  Its sum is a pair of
+            // halves in the lane group's slot 2 * (sub-block % 2) of the row's sums operand,
+            // [64-row group][super-block][M tile][lane][8 halves], the upper four halves zero.
+            sm += __shfl_xor(sm, 1);
+            sm += __shfl_xor(sm, 2);
+            if ((i & 3) == 0) {
+                const float v = sm * (1.0f / (1 << kXBlockSumLog2));
+                const _Float16 vh = (_Float16)v;
+                const _Float16 vl = (_Float16)(__builtin_isinf(v) ? 0.f : v - (float)vh);
+                const int sub = (k >> 5) & 7;
+                _Float16* sd = reinterpret_cast<_Float16*>(a.xsum) +
+                               (((row0 >> 2) + (k >> 8)) * 4 + tile) * 512 + ((sub >> 1) * 16 + m) * 8;
+                *reinterpret_cast<h2*>(sd + 2 * (sub & 1)) = h2{vh, vl};
+                *reinterpret_cast<h2*>(sd + 4 + 2 * (sub & 1)) = h2{(_Float16)0.f, (_Float16)0.f};
+            }
+        }
+    };
+    if (held) {
+#pragma unroll
+        for (int j = 0; j < kHeld; ++j) {
+            const int i = t + kMmThreads * j;
+            if (i < np) put(i, hv[j][0], hv[j][1]);
+        }
+    } else {
+        for (int i = t; i < np; i += kMmThreads) put(i, xr[2 * i], xr[2 * i + 1]);
+    }
+    if (t == 0) {
+        const bool plain = WT == kWeightF32 && (mx > FLT_MAX || (mx > 0.f && ex - 13 < -126));
+        a.xexp[z * a.batch + b] = e + (plain ? kXPlain : 0);
+    }
+}
+
+// The wave's weights, by units of kUnit chunks (F32 one, Q8_0 two, the K-quants a
+// super-block).  fetch(c) loads the unit that holds chunk c, turn() makes the
+// fetched unit the one in hand, expand<CC>() its chunk CC's operands.
+//
+// Quantized types: read straight into the operand layout (16 rows x 4 lane
+// groups a few words each) one load instruction touches 16 rows' lines and the
+// L1's line rate, not the matrix cores, bounds the product (Q8_0 512 x 4096 x
+// 4096 was 46 cycles of L1 per load).  So a fetch loads a tile's 16 rows in
+// 16-byte (Q8_0 8-byte) pieces in row order, and turn() passes them through a
+// few KB of LDS that belong to the wave alone: no barrier, LDS serves a wave's
+// accesses in order.
+typedef uint32_t u2v __attribute__((ext_vector_type(2)));
+typedef uint32_t u3v __attribute__((ext_vector_type(3)));
+
+__device__ __forceinline__ h2 splat2(_Float16 v) { return h2{v, v}; }
+
+template <int WT>
+struct TileW;
+
+constexpr int kTileNT = 2;       // N tiles of a wave
+constexpr int kTurnBytes = 3456;  // LDS of one wave's turn(), the largest type's
+
+struct TileWBase {
+    __amdgpu_buffer_rsrc_t rsrc;
+    int rows;              // rows of the wave inside out_dim (at least one)
+    int n, g, lane;
+    uint32_t* lds;         // the wave's kTurnBytes
+    h8 w[kTileNT][2];      // [N tile][block of the chunk]
+    float d[kTileNT];      // the chunk's scale
+
+    // Rows past out_dim read row out_dim - 1; their sums are never stored.  The
+    // descriptor starts and ends at dwords (Q6_K rows need not): the up to two
+    // bytes this adds at either end share a dword with bytes of the rows.
+    __device__ __forceinline__ int base_init(const MatmulArgs& a, int o0, int64_t row_bytes, int lane_, uint32_t* lds_) {
+        const int first = min(o0, a.out_dim - 1);
+        rows = min(16 * kTileNT, a.out_dim - first);
+        const uintptr_t at = reinterpret_cast<uintptr_t>(a.w) + first * row_bytes;
+        const int skew = (int)(at & 3);
+        rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(at - skew), (short)0,
+                                                 ((int)(rows * row_bytes) + skew + 3) & ~3, 0x00020000);
+        lane = lane_;
+        n = lane & 15;
+        g = lane >> 4;
+        lds = lds_;
+        return skew;
+    }
+    // Piece q of 16 rows of P pieces each, for the lane's i-th load (past the last: the last again).
+    template <int P>
+    __device__ __forceinline__ void piece(int i, int& q, int& row, int& at) const {
+        q = min(lane + 64 * i, 16 * P - 1);
+        row = q / P;
+        at = q - row * P;
+    }
+};
+
+// A unit is two chunks, 136 contiguous bytes of a row (17 pieces of 8).  When
+// the row ends inside it the rest belongs to the next row and is not used.
+template <>
+struct TileW<kWeightQ8_0> : TileWBase {
+    static constexpr bool kLo = false;
+    static constexpr int kUnit = 2, kPieces = 5, kLoads = kPieces * kTileNT;
+    u2v next[kTileNT][kPieces];
+    int off[kTileNT][kPieces], dst[kPieces];
+    struct Raw {
+        uint32_t r0[3], r1[2], s0, s1;
+    } raw[kTileNT][kUnit];
+    float d1[kTileNT];  // block 1's scale (d: block 0's)
+
+    __device__ __forceinline__ void init(const MatmulArgs& a, int o0, int lane_, uint32_t* lds_) {
+        const int row_bytes = (a.in_dim / 32) * 34;
+        base_init(a, o0, row_bytes, lane_, lds_);
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+            int q, row, at;
+            piece<17>(i, q, row, at);
+            dst[i] = 2 * q;
+#pragma unroll
+            for (int j = 0; j < kTileNT; ++j) off[j][i] = min(16 * j + row, rows - 1) * row_bytes + 8 * at;
+        }
+    }
+    __device__ __forceinline__ void fetch(int c) {
+#pragma unroll
+        for (int j = 0; j < kTileNT; ++j)
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) next[j][i] = __builtin_amdgcn_raw_buffer_load_b64(rsrc, off[j][i], c * 68, 0);
+    }
+    // Chunk h of the unit: dwords 17 h .. of the row; block 0's values from byte 2
+    // of dword 2 g on, block 1's at dwords 9 + 2 g and 10 + 2 g, the scales the low half of dword
+    // 0 and the high half of dword 8.
+    __device__ __forceinline__ void turn() {
+#pragma unroll
+        for (int j = 0; j < kTileNT; ++j) {
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) *reinterpret_cast<u2v*>(lds + dst[i]) = next[j][i];
+#pragma unroll
+            for (int h = 0; h < kUnit; ++h) {
+                const uint32_t* row = lds + 34 * n + 17 * h;
+                Raw& r = raw[j][h];
+#pragma unroll
+                for (int i = 0; i < 3; ++i) r.r0[i] = row[2 * g + i];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) r.r1[i] = row[9 + 2 * g + i];
+                r.s0 = row[0];
+                r.s1 = row[8];
+            }
+        }
+    }
+    template <int CC>
+    __device__ __forceinline__ void expand() {
+#pragma unroll
+        for (int j = 0; j < kTileNT; ++j) {
+            const Raw& q = raw[j][CC];
+            w[j][0] = q8_to_h8(__builtin_amdgcn_alignbyte(q.r0[1], q.r0[0], 2), __builtin_amdgcn_alignbyte(q.r0[2], q.r0[1], 2));
+            w[j][1] = q8_to_h8(q.r1[0], q.r1[1]);
+            d[j] = (float)__builtin_bit_cast(_Float16, (uint16_t)(q.s0 & 0xFFFFu));
+            d1[j] = (float)__builtin_bit_cast(_Float16, (uint16_t)(q.s1 >> 16));
+        }
+    }
+};
+
+template <>
+struct TileW<kWeightQ4_K> : TileWBase {
+    static constexpr bool kLo = false;
+    static constexpr int kUnit = 4, kPieces = 3, kLoads = kPieces * kTileNT;
+    u4 next[kTileNT][kPieces];
+    int off[kTileNT][kPieces], dst[kPieces];
+    struct Raw {
+        u4 hd, q[2];
+    } raw[kTileNT];
+    h2 sp[kTileNT];     // the quarter's two scales
+    h2 mp[kTileNT];     // and mins
+    float dm[kTileNT];  // dmin, times 2^6 for the sums' scale
+
+    __device__ __forceinline__ void init(const MatmulArgs& a, int o0, int lane_, uint32_t* lds_) {
+        const int row_bytes = (a.in_dim / 256) * 144;
+        base_init(a, o0, row_bytes, lane_, lds_);
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+            int q, row, at;
+            piece<9>(i, q, row, at);
+            dst[i] = 4 * q;
+#pragma unroll
+            for (int j = 0; j < kTileNT; ++j) off[j][i] = min(16 * j + row, rows - 1) * row_bytes + 16 * at;
+        }
+    }
+    __device__ __forceinline__ void fetch(int c) {
+#pragma unroll
+        for (int j = 0; j < kTileNT; ++j)
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i)
+                next[j][i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[j][i], (c >> 2) * 144, 0);
+    }
+    __device__ __forceinline__ void turn() {
+#pragma unroll
+        for (int j = 0; j < kTileNT; ++j) {
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) *reinterpret_cast<u4*>(lds + dst[i]) = next[j][i];
+            const u4* row = reinterpret_cast<const u4*>(lds) + 9 * n;
+            raw[j].hd = row[0];
+            raw[j].q[0] = row[1 + 2 * g];
+            raw[j].q[1] = row[2 + 2 * g];
+        }
+    }
+    // Chunk CC: sub-block 2 g + CC % 2 (the low or the high nibbles), quant bytes 16 (CC / 2) .. of the quarter.
+    // The operand is sc (q - 8): half the size of sc q, and so is the error of its sums; the 8 sc joins the min term.
+    template <int CC>
+    __device__ __forceinline__ void expand() {
+#pragma unroll
+        for (int j = 0; j < kTileNT; ++j) {
+            const Raw& q = raw[j];
+            if constexpr (CC == 0) {
+                // Sub-blocks 2 g and 2 g + 1: bytes j and j + 4 of the packed scales for g < 2,
+                // else nibbles of byte j + 4 under the top bits of bytes j - 4 and j.
+                const int sh = 16 * (g & 1);
+                const uint32_t b0 = q.hd[1] >> sh, b1 = q.hd[2] >> sh, b2 = q.hd[3] >> sh;
+                const bool low = g < 2;
+                const uint32_t s = low ? b0 & 0x3F3Fu : (b2 & 0x0F0Fu) | ((b0 >> 2) & 0x3030u);
+                const uint32_t m = low ? b1 & 0x3F3Fu : ((b2 >> 4) & 0x0F0Fu) | ((b1 >> 2) & 0x3030u);
+                sp[j] = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, s, 0x04010400u)) - splat2((_Float16)1024.0f);
+                mp[j] = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, m, 0x04010400u)) - splat2((_Float16)1024.0f);
+                d[j] = (float)__builtin_bit_cast(_Float16, (uint16_t)(q.hd[0] & 0xFFFFu));
+                dm[j] = (float)__builtin_bit_cast(_Float16, (uint16_t)(q.hd[0] >> 16)) * (float)(1 << kXBlockSumLog2);
+            }
+            const h2 s2 = splat2(sp[j][CC & 1]);
+            const h2 off8 = s2 * splat2((_Float16)-136.0f);  // exact: a multiple of 8 below 2^14
+#pragma unroll
+            for (int blk = 0; blk < 2; ++blk) {
+                h8 r;
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    // The half 0x5800 | 8 q is 128 + q.
+                    const uint32_t qw = q.q[CC >> 1][2 * blk + t];
+                    const uint32_t u = (CC & 1 ? qw >> 1 : qw << 3) & 0x78787878u;
+                    const h2 p0 = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x58585858u, u, 0x04010400u));
+                    const h2 p1 = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x58585858u, u, 0x04030402u));
+                    const h2 w0 = __builtin_elementwise_fma(p0, s2, off8);  // (128 + q) sc - 136 sc, exact
+                    const h2 w1 = __builtin_elementwise_fma(p1, s2, off8);
+                    r[4 * t + 0] = w0[0];
+                    r[4 * t + 1] = w0[1];
+                    r[4 * t + 2] = w1[0];
+                    r[4 * t + 3] = w1[1];
+                }
+                w[j][blk] = r;
+            }
+        }
+    }
+};
+
+// Super-blocks are 210 bytes, so a row's may start in the middle of a dword: the
+// 53 dwords that hold it are fetched as 13 pieces of 16 bytes and a tail dword,
+// and turn() shifts the lane's words into place.
+template <>
+struct TileW<kWeightQ6_K> : TileWBase {
+    static constexpr bool kLo = true;
+    static constexpr int kUnit = 4, kPieces = 4, kLoads = (kPieces + 1) * kTileNT;
+    u4 next[kTileNT][kPieces];
+    uint32_t tail[kTileNT];
+    int sb_bytes = 0;  // byte offset of the fetched super-block in a row
+    int off[kTileNT][kPieces], dst[kPieces], at16[kPieces];
+    int row_off[kTileNT];  // of row n
+    struct Raw {
+        uint32_t l[2][4], h[4], sc[2], dh;
+    } raw[kTileNT];
+    h8 lo[kTileNT][2];
+
+    __device__ __forceinline__ void init(const MatmulArgs& a, int o0, int lane_, uint32_t* lds_) {
+        const int row_bytes = (a.in_dim / 256) * 210;
+        const int skew = base_init(a, o0, row_bytes, lane_, lds_);
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+            int q, row;
+            piece<13>(i, q, row, at16[i]);
+            dst[i] = 4 * q;
+#pragma unroll
+            for (int j = 0; j < kTileNT; ++j) off[j][i] = skew + min(16 * j + row, rows - 1) * row_bytes;
+        }
+#pragma unroll
+        for (int j = 0; j < kTileNT; ++j) row_off[j] = skew + min(16 * j + n, rows - 1) * row_bytes;
+    }
+    __device__ __forceinline__ void fetch(int c) {
+        const int sb = (c >> 2) * 210;
+        sb_bytes = sb;
+#pragma unroll
+        for (int j = 0; j < kTileNT; ++j) {
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i)
+                next[j][i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, ((off[j][i] + sb) & ~3) + 16 * at16[i], 0, 0);
+            tail[j] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, ((row_off[j] + sb) & ~3) + 208, 0, 0);
+        }
+    }
+    __device__ __forceinline__ void turn() {
+        const int hn = g >> 1, l = 4 * (g & 1);  // half of the super-block, the lane's dwords in a quarter
+#pragma unroll
+        for (int j = 0; j < kTileNT; ++j) {
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) *reinterpret_cast<u4*>(lds + dst[i]) = next[j][i];
+            const uint32_t* row = lds + 52 * n;
+            const int s = (row_off[j] + sb_bytes) & 2;
+            auto window = [&](int at, uint32_t (&out)[4]) {
+                const u4 v = *reinterpret_cast<const u4*>(row + at);
+                const uint32_t e = row[at + 4];
+                out[0] = __builtin_amdgcn_alignbyte(v[1], v[0], s);
+                out[1] = __builtin_amdgcn_alignbyte(v[2], v[1], s);
+                out[2] = __builtin_amdgcn_alignbyte(v[3], v[2], s);
+                out[3] = __builtin_amdgcn_alignbyte(e, v[3], s);
+            };
+            Raw& r = raw[j];
+            window(16 * hn + l, r.l[0]);
+            window(16 * hn + l + 8, r.l[1]);
+            window(32 + 8 * hn + l, r.h);
+            const uint32_t s0 = row[48 + 2 * hn], s1 = row[49 + 2 * hn];
+            const uint32_t s2 = hn ? tail[j] : row[50];
+            r.sc[0] = __builtin_amdgcn_alignbyte(s1, s0, s);
+            r.sc[1] = __builtin_amdgcn_alignbyte(s2, s1, s);
+            r.dh = tail[j] >> (8 * s);  // d in the low half
+        }
+    }
+    // Chunk CC is quarter CC of the half: its 16 values of the lane share the scale 8 n + g % 2 + 2 CC.
+    template <int CC>
+    __device__ __forceinline__ void expand() {
+#pragma unroll
+        for (int j = 0; j < kTileNT; ++j) {
+            const Raw& r = raw[j];
+            if constexpr (CC == 0) d[j] = (float)__builtin_bit_cast(_Float16, (uint16_t)(r.dh & 0xFFFFu));
+            const int sv = (int)(int8_t)((r.sc[CC >> 1] >> (8 * (g & 1) + 16 * (CC & 1))) & 0xFFu);
+            const h2 s2 = splat2((_Float16)(float)sv);
+#pragma unroll
+            for (int blk = 0; blk < 2; ++blk) {
+                h8 hi, lw;
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const uint32_t u = ((r.l[CC & 1][2 * blk + t] >> (4 * (CC >> 1))) & 0x0F0F0F0Fu) |
+                                       (((r.h[2 * blk + t] >> (2 * CC)) & 0x03030303u) << 4);
+                    h2 q[2];
+                    six_to_h4(u, q[0], q[1]);
+#pragma unroll
+                    for (int v = 0; v < 2; ++v) {
+                        const h2 m = q[v] * s2;
+                        const h2 rest = __builtin_elementwise_fma(q[v], s2, -m);  // exact: 0 or +-1
+                        hi[4 * t + 2 * v] = m[0];
+                        hi[4 * t + 2 * v + 1] = m[1];
+                        lw[4 * t + 2 * v] = rest[0];
+                        lw[4 * t + 2 * v + 1] = rest[1];
+                    }
+                }
+                w[j][blk] = hi;
+                lo[j][blk] = lw;
+            }
+        }
+    }
+};
+
+// Max of x over lanes l, l ^ 16, l ^ 32 and l ^ 48.
+__device__ __forceinline__ float lane_group_max(float x) {
+    const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
+    const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r32[0]), __uint_as_float(r32[1]));
+}
+
+// One chunk per unit, fetched two ahead straight into the operand layout (a load
+// covers 64 contiguous bytes of each row).
+template <>
+struct TileW<kWeightF32> : TileWBase {
+    static constexpr bool kLo = true;
+    static constexpr int kUnit = 1, kLoads = 4 * kTileNT;
+    struct Raw {
+        f4 v[4];
+    } next[2][kTileNT];
+    int row_off[kTileNT];
+    h8 lo[kTileNT][2];
+    uint32_t plain = 0;  // bit j: row j has a chunk the fp16 pairs cannot stand for (see below)
+
+    __device__ __forceinline__ void init(const MatmulArgs& a, int o0, int lane_, uint32_t* lds_) {
+        base_init(a, o0, (int64_t)a.in_dim * 4, lane_, lds_);
+#pragma unroll
+        for (int j = 0; j < kTileNT; ++j) row_off[j] = min(16 * j + n, rows - 1) * a.in_dim * 4 + 16 * g;
+    }
+    __device__ __forceinline__ void fetch(int slot, int c) {
+#pragma unroll
+        for (int j = 0; j < kTileNT; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                next[slot][j].v[i] =
+                    __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, row_off[j] + 64 * i, c * 256, 0));
+    }
+    // The row's largest |w| of the chunk goes to [2^12, 2^13).  d is 2^(e - 13), the
+    // other 2^13 joining the batch row's exponent at the end, so that the running
+    // sum stays about |w| times the scaled x.  Chunks that reach 2^100 (or hold an infinity), or
+    // whose largest is below 2^-100, leave fp16's or that sum's range: their row is summed in plain fp32.
+    template <int CC>
+    __device__ __forceinline__ void expand(int slot) {
+#pragma unroll
+        for (int j = 0; j < kTileNT; ++j) {
+            const f4 (&r)[4] = next[slot][j].v;
+            float mx = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                mx = fmaxf(mx, fmaxf(fmaxf(fabsf(r[i][0]), fabsf(r[i][1])), fmaxf(fabsf(r[i][2]), fabsf(r[i][3]))));
+            mx = lane_group_max(mx);
+            const int field = (int)(__float_as_uint(mx) >> 23);
+            const int e = min(87, max(-113, field - 139));  // field 126 + ex, mx = f * 2^ex with f in [0.5, 1)
+            if (mx > 0.f && (field - 139 > 87 || field - 139 < -113)) plain |= 1u << j;
+            const float down = __uint_as_float((uint32_t)(127 - e) << 23);
+            d[j] = __uint_as_float((uint32_t)(127 + e - 13) << 23);
+#pragma unroll
+            for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const float v = r[2 * blk + (q >> 2)][q & 3] * down;
+                    const _Float16 hi = (_Float16)v;
+                    w[j][blk][q] = hi;
+                    lo[j][blk][q] = (_Float16)(v - (float)hi);
+                }
+        }
+    }
+};
+
+// x in LDS: a ring of four chunks, each an array of its own so that the
+// compiler sees which direct loads a read depends on.
+struct TileLds {
+    u4 *x0, *x1, *x2, *x3;
+    template <int S>
+    __device__ __forceinline__ u4* slot() const {
+        return S == 0 ? x0 : S == 1 ? x1 : S == 2 ? x2 : x3;
+    }
+};
+
+// The workgroup's K loop over MT M tiles (16 MT batch rows from 64 by).
+//
+// Per chunk c the direct loads of x chunk c + 3 go out, and at a unit's start the
+// fetch of the next unit (F32: of chunk c + 2), then chunk c's products run.  A
+// wave waits for its part of chunk c + 1 before the barrier that ends chunk c.
+// Memory loads count in order, so it waits until only the loads issued after
+// that part are left: the 2 MT direct loads of chunks c + 2 and c + 3, and those
+// of the fetches in chunks c - 2 .. c (the compiler may not move loads over the
+// asm).  Past the range's end the last chunk is loaded again (into a slot nobody
+// reads any more), so that the count holds to the end.
+template <int WT, int MT>
+__device__ __forceinline__ void tile_products(const MatmulArgs& a, TileW<WT>& w, f4 (&acc)[4][kTileNT], const TileLds& xs,
+                                              int by, int c_begin, int c_end) {
+    constexpr int NT = kTileNT;
+    constexpr int kUnit = TileW<WT>::kUnit;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int chunks = a.in_dim / 64;
+
+    // The 4 MT KB of a chunk's M tiles: wave w moves kilobytes w MT .. + MT - 1.
+    const _Float16* xg = static_cast<const _Float16*>(a.xh) + (int64_t)by * chunks * 4 * kTileHalves;
+    auto stage_x = [&](auto s_t, int c) {
+        u4* dst = xs.slot<decltype(s_t)::value>();
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<_Float16*>(xg + (int64_t)min(c, c_end - 1) * 4 * kTileHalves), (short)0, 4 * kTileHalves * 2, 0x00020000);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                r, (__attribute__((address_space(3))) void*)(dst + 64 * (wave * MT + i)), 16, 16 * lane,
+                1024 * (wave * MT + i), 0, 0);
+    };
+    // Q4_K: the M tiles' sub-block sums of a super-block.
+    const h8* sg = reinterpret_cast<const h8*>(a.xsum) + (int64_t)by * (chunks / 4) * 256 + lane;
+    h8 sx[MT];
+    auto load_sums = [&](int c) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) sx[t] = sg[(c >> 2) * 256 + 64 * t];
+    };
+
+    // Chunk c = c_begin + S (mod 4).
+    auto chunk = [&](auto s_t, int c) {
+        constexpr int S = decltype(s_t)::value;
+        constexpr int CC = S % kUnit;
+        stage_x(std::integral_constant<int, (S + 3) % 4>{}, c + 3);
+        if constexpr (WT == kWeightF32) {
+            w.template expand<CC>(S % 2);
+            w.fetch(S % 2, min(c + 2, c_end - 1));
+        } else {
+            // The last unit once more at the range's end, unused.
+            if constexpr (CC == 0) w.fetch(c + kUnit < c_end ? c + kUnit : c);
+            w.template expand<CC>();
+        }
+        if constexpr (WT == kWeightQ4_K) {
+            if constexpr (CC == 0) {  // the super-block's min term, dmin m - 8 d sc against the sums of x
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    const h8 mb = h8{w.mp[j][0], w.mp[j][0], w.mp[j][1], w.mp[j][1], 0, 0, 0, 0};
+                    const h8 sb = h8{w.sp[j][0], w.sp[j][0], w.sp[j][1], w.sp[j][1], 0, 0, 0, 0};
+                    const float d8 = w.d[j] * (float)(8 << kXBlockSumLog2);
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) {
+                        const f4 pm = __builtin_amdgcn_mfma_f32_16x16x32_f16(sx[t], mb, f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                        const f4 ps = __builtin_amdgcn_mfma_f32_16x16x32_f16(sx[t], sb, f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            acc[t][j][r] = fmaf(-w.dm[j], pm[r], fmaf(d8, ps[r], acc[t][j][r]));
+                    }
+                }
+                load_sums(min(c + 4, c_end - 1));
+            }
+        }
+        const h8* xb = reinterpret_cast<const h8*>(xs.slot<S>()) + lane;
+        // M tiles in pairs: 2 NT independent accumulator chains keep the matrix
+        // cores busy through each other's latency.
+        constexpr int kPair = MT < 2 ? 1 : 2;
+#pragma unroll
+        for (int t0 = 0; t0 < MT; t0 += kPair) {
+            h8 ax[kPair][2][2];
+#pragma unroll
+            for (int p = 0; p < kPair; ++p)
+#pragma unroll
+                for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) ax[p][blk][h] = xb[(t0 + p) * (kTileHalves / 8) + (blk * 2 + h) * 64];
+            f4 part[kPair][NT], sum[kPair][NT];
+            auto zero = [&] {
+#pragma unroll
+                for (int p = 0; p < kPair; ++p)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) part[p][j] = f4{0.f, 0.f, 0.f, 0.f};
+            };
+            auto step = [&](int blk, int h, const h8 (&wv)[NT][2]) {
+#pragma unroll
+                for (int p = 0; p < kPair; ++p)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+                        part[p][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ax[p][blk][h], wv[j][blk], part[p][j], 0, 0, 0);
+            };
+            auto add = [&](const float (&sc)[NT]) {
+#pragma unroll
+                for (int p = 0; p < kPair; ++p)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[t0 + p][j][r] = fmaf(sc[j], part[p][j][r], acc[t0 + p][j][r]);
+            };
+            zero();
+#pragma unroll
+            for (int blk = 0; blk < 2; ++blk) {
+                step(blk, 1, w.w);
+                if constexpr (TileW<WT>::kLo) step(blk, 0, w.lo);
+                step(blk, 0, w.w);
+                if constexpr (WT == kWeightQ8_0) {
+                    // Each block its own scale; the chunk's two sums join before the running
+                    // one, which then rounds once a chunk as for the other types.
+#pragma unroll
+                    for (int p = 0; p < kPair; ++p)
+#pragma unroll
+                        for (int j = 0; j < NT; ++j)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                if (blk == 0) sum[p][j][r] = w.d[j] * part[p][j][r];
+                                else acc[t0 + p][j][r] += fmaf(w.d1[j], part[p][j][r], sum[p][j][r]);
+                            }
+                    zero();
+                }
+            }
+            if constexpr (WT != kWeightQ8_0) add(w.d);
+        }
+        if constexpr (WT != kWeightF32) {
+            if constexpr (CC == kUnit - 1) w.turn();
+        }
+        // lgkmcnt(0): this wave's reads of the slot are done, and the next chunk's direct loads may overwrite it.
+        constexpr int kFetches = (S % kUnit == 0) + ((S + 3) % kUnit == 0) + ((S + 2) % kUnit == 0);
+        constexpr int kLater = 2 * MT + kFetches * (TileW<WT>::kLoads + (WT == kWeightQ4_K ? MT : 0));
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kLater) : "memory");
+        __builtin_amdgcn_s_barrier();
+    };
+
+    if constexpr (WT == kWeightF32) {
+        w.fetch(0, c_begin);
+        w.fetch(1, min(c_begin + 1, c_end - 1));
+    } else {
+        w.fetch(c_begin);
+    }
+    if constexpr (WT == kWeightQ4_K) load_sums(c_begin);
+    stage_x(std::integral_constant<int, 0>{}, c_begin);
+    stage_x(std::integral_constant<int, 1>{}, c_begin + 1);
+    stage_x(std::integral_constant<int, 2>{}, c_begin + 2);
+    if constexpr (WT != kWeightF32) w.turn();
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // chunks c_begin .. + 2 have landed
+    __builtin_amdgcn_s_barrier();
+    for (int c = c_begin; c < c_end; c += 4) {  // super-block types: ranges are whole super-blocks (host)
+        chunk(std::integral_constant<int, 0>{}, c);
+        if (kUnit < 4 && c + 1 >= c_end) break;
+        chunk(std::integral_constant<int, 1>{}, c + 1);
+        if (kUnit < 4 && c + 2 >= c_end) break;
+        chunk(std::integral_constant<int, 2>{}, c + 2);
+        if (kUnit < 4 && c + 3 >= c_end) break;
+        chunk(std::integral_constant<int, 3>{}, c + 3);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load outlives the loop
+}
+
+template <int WT>
+__global__ __launch_bounds__(kMmThreads, 2) void matmul_tile_kernel(MatmulArgs a) {
+    constexpr int NT = kTileNT;
+    __shared__ u4 xs0[4 * kTileHalves / 8], xs1[4 * kTileHalves / 8], xs2[4 * kTileHalves / 8], xs3[4 * kTileHalves / 8];
+    __shared__ u4 turn[4][kTurnBytes / 16];
+    const TileLds xs{xs0, xs1, xs2, xs3};
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15;
+    const int g = lane >> 4;
+    const int chunks = a.in_dim / 64;
+
+    // Workgroups go to the eight XCDs in turn; each XCD takes a contiguous run of
+    // (range, weight tile, batch group), batch groups fastest, so that the
+    // workgroups that share a weight tile share an L2.
+    const int wtiles = (a.out_dim + 64 * NT - 1) / (64 * NT);
+    const int groups = (a.batch + 63) / 64;
+    const int total = wtiles * groups * a.splits;
+    const int xcd = blockIdx.x % 8, per_xcd = total / 8, extra = total % 8;
+    const int id = xcd * per_xcd + min(xcd, extra) + blockIdx.x / 8;
+    const int by = id % groups;
+    const int bx = (id / groups) % wtiles;
+    const int z = id / (groups * wtiles);
+
+    const int b0 = by * 64;
+    const int mt = min(4, (a.batch - b0 + 15) >> 4);  // M tiles in use
+    const int o0 = (bx * 4 + wave) * 16 * NT;
+    const int c_begin = z * a.chunks_per_split;
+    const int c_end = min(chunks, c_begin + a.chunks_per_split);
+
+    TileW<WT> w;
+    w.init(a, o0, lane, reinterpret_cast<uint32_t*>(turn[wave]));
+    f4 acc[4][NT];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[t][j] = f4{0.f, 0.f, 0.f, 0.f};
+    if (mt > 2) tile_products<WT, 4>(a, w, acc, xs, by, c_begin, c_end);
+    else if (mt == 2) tile_products<WT, 2>(a, w, acc, xs, by, c_begin, c_end);
+    else tile_products<WT, 1>(a, w, acc, xs, by, c_begin, c_end);
+
+    // Lane holds batch rows b0 + 16 t + 4 g + r of weight rows o0 + 16 j + n.
+    float* dst = a.split_out ? a.split_out + (int64_t)z * a.batch * a.out_dim : a.y;
+    constexpr int kExtra = WT == kWeightF32 ? 13 : 0;
+    bool plain_any = false;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int b = b0 + 16 * t + 4 * g + r;
+            if (b >= a.batch) continue;
+            const int e = a.xexp[z * a.batch + b];
+            if (WT == kWeightF32 && e > kXPlain / 2) plain_any = true;
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const int o = o0 + 16 * j + n;
+                if (o < a.out_dim) dst[(int64_t)b * a.out_dim + o] = ldexpf(acc[t][j][r], e + kExtra);
+            }
+        }
+    if constexpr (WT == kWeightF32) {
+        // Outputs of rows the fp16 pairs cannot stand for: the same lane's plain sum replaces what it stored.
+        if (plain_any || w.plain) {
+            for (int i = 0; i < 16 * NT; ++i) {
+                const int b = b0 + 16 * (i & 3) + 4 * g + ((i >> 2) & 3);
+                const int j = i >> 4;
+                const int o = o0 + 16 * j + n;
+                if (b >= a.batch || o >= a.out_dim) continue;
+                if (a.xexp[z * a.batch + b] <= kXPlain / 2 && !((w.plain >> j) & 1)) continue;
+                const float* wr = static_cast<const float*>(a.w) + (int64_t)o * a.in_dim;
+                const float* xr = a.x + (int64_t)b * a.in_dim;
+                float s = 0.f;
+                for (int k = 64 * c_begin; k < 64 * c_end; ++k) s = fmaf(wr[k], xr[k], s);
+                dst[(int64_t)b * a.out_dim + o] = s;
+            }
+        }
+    }
+}
+
 // y = the sum over z of the split partials, in z order; four elements per
 // thread and step when y and the partials are 16-byte aligned, else one.
 __global__ __launch_bounds__(kMmThreads) void matmul_reduce_kernel(MatmulArgs a) {
@@ -1370,6 +2185,39 @@ hipError_t launch_matmul_small(const MatmulArgs& a, hipStream_t stream) {
     return hipGetLastError();
 }
 
+int matmul_tile_rows() { return 64 * kTileNT; }
+
+static void launch_reduce(const MatmulArgs& a, hipStream_t stream) {
+    const int64_t n = (int64_t)a.batch * a.out_dim;
+    const int blocks = (int)std::min<int64_t>((n / 4 + kMmThreads - 1) / kMmThreads + 1, 2048);
+    hipLaunchKernelGGL(matmul_reduce_kernel, dim3(blocks), dim3(kMmThreads), 0, stream, a);
+}
+
+// The tile form: the x pre-pass, then matmul_tile_kernel.
+hipError_t launch_matmul_tile(const MatmulArgs& a, hipStream_t stream) {
+    if (a.batch <= 0 || a.out_dim <= 0) return hipSuccess;
+    const bool kquant = a.w_type == kWeightQ4_K || a.w_type == kWeightQ6_K;
+    if (!a.xh || !a.xexp || a.chunks_per_split < 1 || (a.splits > 1) != (a.split_out != nullptr) ||
+        (kquant && (a.in_dim % 256 != 0 || a.chunks_per_split % 4 != 0)) || (a.w_type == kWeightQ4_K && !a.xsum))
+        return hipErrorInvalidValue;
+    const int64_t total = (int64_t)((a.out_dim + 64 * kTileNT - 1) / (64 * kTileNT)) * ((a.batch + 63) / 64) * a.splits;
+    if (total > INT32_MAX) return hipErrorInvalidValue;
+    auto go = [&](auto wt) {
+        constexpr int WT = decltype(wt)::value;
+        hipLaunchKernelGGL(matmul_split_x_tile_kernel<WT>, dim3(a.batch, a.splits), dim3(kMmThreads), 0, stream, a);
+        hipLaunchKernelGGL(matmul_tile_kernel<WT>, dim3((unsigned)total), dim3(kMmThreads), 0, stream, a);
+        if (a.splits > 1) launch_reduce(a, stream);
+        return hipGetLastError();
+    };
+    switch (a.w_type) {
+        case kWeightF32: return go(std::integral_constant<int, kWeightF32>{});
+        case kWeightQ8_0: return go(std::integral_constant<int, kWeightQ8_0>{});
+        case kWeightQ4_K: return go(std::integral_constant<int, kWeightQ4_K>{});
+        case kWeightQ6_K: return go(std::integral_constant<int, kWeightQ6_K>{});
+    }
+    return hipErrorInvalidValue;
+}
+
 hipError_t launch_matmul(const MatmulArgs& a, hipStream_t stream) {
     if (a.batch <= 0 || a.out_dim <= 0) return hipSuccess;
     const dim3 grid((a.out_dim + kMmRowsWg - 1) / kMmRowsWg, (a.batch + 63) / 64, a.splits);
@@ -1392,11 +2240,7 @@ hipError_t launch_matmul(const MatmulArgs& a, hipStream_t stream) {
         hipLaunchKernelGGL(matmul_batch_kernel<kWeightQ6_K>, grid, dim3(kMmThreads), 0, stream, a);
     else
         return hipErrorInvalidValue;
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || a.splits <= 1) return e;
-    const int64_t n = (int64_t)a.batch * a.out_dim;
-    const int blocks = (int)std::min<int64_t>((n / 4 + kMmThreads - 1) / kMmThreads + 1, 2048);
-    hipLaunchKernelGGL(matmul_reduce_kernel, dim3(blocks), dim3(kMmThreads), 0, stream, a);
+    if (a.splits > 1) launch_reduce(a, stream);
     return hipGetLastError();
 }
 

@@ -878,6 +878,36 @@ constexpr int64_t kMatmulF16MinOutputs = 196608;
 // Q4_K 17.0 -> 17.25 us, Q6_K 18.6 -> 19.1 us, while Q8_0 gains 16.8 -> 15.8).
 constexpr int64_t kMatmulSmallMinOutputs = 16384;
 
+// Which products take the tile form (gsp_matmul.hip): those with enough work to
+// cover its x pre-pass and its long pipeline.  Measured against the form each
+// size took before (us, before -> after; in x out at rows):
+//   Q4_K above 64 rows: 4096 x 4096 at 1024 185 -> 102, at 100 34.7 -> 28.9,
+//     4096 x 16384 at 65 76 -> 52, 1024 x 1024 at 3000 46 -> 42; below the line
+//     3584 x 3584 at 65 27.6 -> 27.6, 3584 x 512 at 2048 59 -> 64.
+//   Q4_K up to 64 rows, by the weights alone: 4096 x 32768 at 16 68 -> 31, 3584
+//     x 18944 at 64 58 -> 46, 4096 x 8192 at 33 29.7 -> 28.2; below 4096 x 6144 at 48 27.1 -> 27.8,
+//     4096 x 4096 at 64 21.8 -> 24.3.
+//   Q8_0 above 64 rows: 4096 x 4096 at 1024 177 -> 113, 3584 x 3584 at 300 56
+//     -> 51; below 128 rows 30.5 -> 32.1.  Up to 64 rows only the widest outputs
+//     gain, at a larger summation error than the small form's, so none take it.
+//   Q6_K above 64 rows: 4096 x 4096 at 1024 194 -> 136, 3584 x 3584 at 300 73
+//     -> 62; 1024 x 4864 at 1000 68.0 -> 68.4, 3584 x 3584 at 128 37 -> 38.5.
+//   F32: 4096 x 4096 at 1024 279 -> 166, at 256 88 -> 59, 3584 x 3584 at 128
+//     46.5 -> 41.3, 18944 x 3584 at 64 114 -> 96; below 4096 x 1024 at 300 37.8
+//     -> 39.7, 4096 x 16384 at 33 76 -> 79.
+static bool use_matmul_tile(int32_t w_type, int64_t in_dim, int64_t out_dim, int64_t batch) {
+    // The kernel's 32-row descriptors and its workgroup index are 32-bit.
+    if (in_dim * 4 * 32 > INT32_MAX || (out_dim + 127) / 128 * ((batch + 63) / 64) > INT32_MAX / 64) return false;
+    const double macs = (double)batch * (double)in_dim * (double)out_dim;
+    switch (w_type) {
+        case GSP_WTYPE_Q4_K: return batch > 64 ? out_dim >= 1024 && macs >= 1.5e9 : in_dim * out_dim >= (1 << 25);
+        case GSP_WTYPE_Q8_0: return batch > 64 && out_dim >= 2048 && macs >= 3e9;
+        case GSP_WTYPE_Q6_K: return batch > 64 && out_dim >= 2048 && in_dim >= 2048 && macs >= 3.5e9;
+        case GSP_WTYPE_F32: return batch > 64 ? out_dim >= 1024 && macs >= 1.5e9 : macs >= 4e9;
+    }
+    return false;
+}
+
 int gsp_matmul_batch(gsp_ctx* ctx, int32_t w_type, const void* w_dev, const float* x_dev, float* y_dev,
                      int32_t in_dim, int32_t out_dim, int32_t batch) {
     gsp::clear_error();
@@ -901,6 +931,43 @@ int gsp_matmul_batch(gsp_ctx* ctx, int32_t w_type, const void* w_dev, const floa
                          (int)walign);
     int rc = set_device(ctx);
     if (rc) return rc;
+    if (use_matmul_tile(w_type, in_dim, out_dim, batch)) {
+        // Splits: K ranges of at least 8 chunks, about one workgroup per CU (4096 x
+        // 4096 at 100 rows Q4_K, 64 tiles: 47.6 us unsplit, 27.4 in 4 ranges, 31.1 in
+        // 8; F32 at 256 rows, 128 tiles: 60 us in 2, 67 in 3, where half the CUs run
+        // two workgroups; 3584 x 18944 at 64 rows Q4_K, 148 tiles: 47.3 and 45.8 in 2;
+        // 4096 x 4096 at 512 rows, 256 tiles, 58.0 and 58.4 in 2; at 1024 rows 100 and 112).
+        const int64_t chunks = in_dim / 64;
+        const int64_t groups = (batch + 63) / 64;
+        const int64_t tiles = groups * ((out_dim + gsp::matmul_tile_rows() - 1) / gsp::matmul_tile_rows());
+        const int64_t unit = kquant ? 4 : 1;  // K-quant ranges are whole super-blocks
+        int64_t splits = std::max<int64_t>(1, 6 * (int64_t)std::max(1, ctx->num_cus) / (5 * tiles));
+        splits = std::min(splits, std::max<int64_t>(1, chunks / 8));
+        int64_t per = (chunks + splits - 1) / splits;
+        per = (per + unit - 1) / unit * unit;
+        splits = (chunks + per - 1) / per;
+        gsp::MatmulArgs a{};
+        a.w = w_dev;
+        a.x = x_dev;
+        a.y = y_dev;
+        a.w_type = w_type;
+        a.in_dim = in_dim;
+        a.out_dim = out_dim;
+        a.batch = batch;
+        a.splits = (int32_t)splits;
+        a.chunks_per_split = (int32_t)per;
+        rc = ensure_device(ctx, &ctx->d_mmx, &ctx->d_mmx_halves, (size_t)groups * 64 * in_dim * 2, false);
+        if (!rc) rc = ensure_device(ctx, &ctx->d_mmexp, &ctx->d_mmexp_words, (size_t)splits * batch, false);
+        if (!rc && splits > 1) rc = ensure_device(ctx, &ctx->d_mm, &ctx->d_mm_floats, (size_t)splits * batch * out_dim, false);
+        if (!rc && w_type == GSP_WTYPE_Q4_K)
+            rc = ensure_device(ctx, &ctx->d_mmxs, &ctx->d_mmxs_floats, (size_t)groups * (in_dim / 256) * 1024, false);
+        if (rc) return rc;
+        a.xh = ctx->d_mmx;
+        a.xexp = ctx->d_mmexp;
+        a.split_out = splits > 1 ? ctx->d_mm : nullptr;
+        a.xsum = w_type == GSP_WTYPE_Q4_K ? ctx->d_mmxs : nullptr;
+        return check_hip(gsp::launch_matmul_tile(a, ctx->stream), "matmul launch");
+    }
     if ((w_type == GSP_WTYPE_Q8_0 || w_type == GSP_WTYPE_Q4_K || w_type == GSP_WTYPE_Q6_K) && batch <= 64 &&
         (int64_t)batch * out_dim >= kMatmulSmallMinOutputs &&
         (in_dim / 64 + gsp::matmul_small_range_chunks_max() - 1) / gsp::matmul_small_range_chunks_max() <=

@@ -267,3 +267,68 @@ def test_kquant_matmul_errors(torch_mod, gsp, ctx):
         ctx.matmul_batch(gsp.WTYPE_Q4_K, w.data_ptr() + 2, x.data_ptr(), y.data_ptr(), 256, 16, 4)
     with pytest.raises(gsp.InvalidArgument):  # Q6_K as 2-byte words
         ctx.matmul_batch(gsp.WTYPE_Q6_K, w.data_ptr() + 1, x.data_ptr(), y.data_ptr(), 256, 16, 4)
+
+
+# The tile form (matmul_tile_kernel), which takes products with enough work: ragged batch groups (one, two
+# and four M tiles in the last), ragged weight tiles, odd chunk counts (Q8_0, F32), super-block rows that
+# start in the middle of a dword (Q6_K with an odd number of super-blocks), split and unsplit K.
+TILE_SHAPES = [
+    # (w_type, in_dim, out_dim, batch)
+    (orc.WTYPE_Q4_K, 4096, 2100, 190),    # split K, last group four M tiles
+    (orc.WTYPE_Q4_K, 256, 17000, 400),    # one super-block, one M tile in the last group
+    (orc.WTYPE_Q4_K, 2048, 16500, 5),     # up to 64 rows: by the weights alone
+    (orc.WTYPE_Q4_K, 2304, 16391, 31),
+    (orc.WTYPE_Q8_0, 1088, 16401, 180),   # 17 chunks: the last unit of two is half a unit
+    (orc.WTYPE_Q8_0, 18944, 2048, 90),    # split K, ranges of odd length
+    (orc.WTYPE_Q6_K, 2304, 8203, 193),    # 9 super-blocks: odd rows are not dword aligned
+    (orc.WTYPE_Q6_K, 5376, 2055, 330),    # split K
+    (orc.WTYPE_F32, 2112, 4099, 200),     # 33 chunks
+    (orc.WTYPE_F32, 64, 32771, 800),      # one chunk
+    (orc.WTYPE_F32, 4096, 16400, 64),
+]
+
+
+@pytest.mark.parametrize("w_type,in_dim,out_dim,batch", TILE_SHAPES, ids=lambda v: str(v))
+def test_tile_form_matches_float64(torch_mod, gsp, ctx, w_type, in_dim, out_dim, batch):
+    print(f"case matmul tile type={w_type} {in_dim}x{out_dim} b{batch}", flush=True)
+    rng = np.random.default_rng(in_dim * 7 + out_dim + batch + w_type)
+    if w_type in (orc.WTYPE_Q4_K, orc.WTYPE_Q6_K):
+        data, wm = _kquant_weights(rng, w_type, out_dim, in_dim)
+    else:
+        data, wm = _weights(rng, w_type, out_dim, in_dim)
+    x = rng.standard_normal((batch, in_dim)).astype(np.float32)
+    got = _run(torch_mod, gsp, ctx, w_type, data, x, in_dim, out_dim)
+    x64 = x.astype(np.float64)
+    wm = wm.astype(np.float64)
+    assert np.all(np.isfinite(got))
+    assert np.all(np.abs(got - x64 @ wm.T) <= 1e-5 * (np.abs(x64) @ np.abs(wm).T) + 1e-7)
+    again = _run(torch_mod, gsp, ctx, w_type, data, x, in_dim, out_dim)
+    assert np.array_equal(got, again)
+
+
+def test_tile_form_f32_beyond_the_fp16_pairs(torch_mod, gsp, ctx):
+    """F32 weights and inputs that no scaled fp16 pair stands for: infinities, NaN, weights of 1e35 and rows
+    of 1e-37.  Those outputs are plain fp32 sums: non-finite exactly where fp32 arithmetic makes them so."""
+    in_dim, out_dim, batch = 1024, 8200, 190
+    rng = np.random.default_rng(5)
+    w = rng.standard_normal((out_dim, in_dim)).astype(np.float32) * np.float32(0.03)
+    x = rng.standard_normal((batch, in_dim)).astype(np.float32)
+    w[3, 100], w[5, 7], w[6, 8] = np.inf, -np.inf, np.nan
+    w[40:60] *= np.float32(1e30)       # finite sums of large weights, one row's largest beyond 2^100
+    w[41, 5] = np.float32(2e35)
+    w[70] *= np.float32(1e-36)         # below the pairs' exponents
+    w[8200 - 1, 1023] = np.inf
+    x[10, 3], x[11, 4], x[189, 1000] = np.inf, np.nan, -np.inf
+    x[20] *= np.float32(1e-37)
+    got = _run(torch_mod, gsp, ctx, orc.WTYPE_F32, w, x, in_dim, out_dim)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = x.astype(np.float64) @ w.astype(np.float64).T
+        # The magnitude of the finite terms; a non-finite reference is compared by kind.
+        mag = np.abs(x.astype(np.float64)) @ np.abs(w.astype(np.float64)).T
+    kinds = np.isfinite(ref)
+    assert np.array_equal(np.isnan(ref), np.isnan(got))
+    assert np.array_equal(np.sign(ref[np.isinf(ref)]), np.sign(got[np.isinf(ref)]))
+    assert np.all(np.isinf(got[np.isinf(ref)]))
+    # fp32 sums of K terms round to 1e-5 of the terms' magnitude at worst; rows of 1e-37 lose their
+    # products below the smallest normal (K terms of half 2^-149 each, and flushed subnormals of 2^-126).
+    assert np.all(np.abs(got[kinds] - ref[kinds]) <= 1e-5 * mag[kinds] + in_dim * 2.0 ** -126)
