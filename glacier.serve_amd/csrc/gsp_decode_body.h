@@ -485,16 +485,65 @@ __device__ __forceinline__ void page_pv(WaveState<D>& st, const PageRegs<D, _Flo
     // i.e. element i of the lane's four V pieces.
     // P arrives times 2^12 (compute_page), so p_lo of a typical probability is a
     // normal fp16 number: the matrix cores flush fp16 subnormals.
+    typedef _Float16 h8 __attribute__((ext_vector_type(8)));
     const h4 ph = __builtin_convertvector(p, h4);
     const h4 pl = __builtin_convertvector(p - __builtin_convertvector(ph, f4), h4);
+    // Both halves in one rank-32 step (it takes the cycles of a rank-16 one): k slots
+    // 8g + 0..3 are p_hi of tokens 4g + 0..3 and 8g + 4..7 their p_lo, against V twice.
+    const h8 pp = __builtin_shufflevector(ph, pl, 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
     for (int c = 0; c < D / 64; ++c)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const h4 b = {pr.v[0][c][i], pr.v[1][c][i], pr.v[2][c][i], pr.v[3][c][i]};
-            st.o[4 * c + i] = __builtin_amdgcn_mfma_f32_16x16x16f16(ph, b, st.o[4 * c + i], 0, 0, 0);
-            st.o[4 * c + i] = __builtin_amdgcn_mfma_f32_16x16x16f16(pl, b, st.o[4 * c + i], 0, 0, 0);
+            const _Float16 v0 = pr.v[0][c][i], v1 = pr.v[1][c][i], v2 = pr.v[2][c][i], v3 = pr.v[3][c][i];
+            const h8 b = {v0, v1, v2, v3, v0, v1, v2, v3};
+            st.o[4 * c + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pp, b, st.o[4 * c + i], 0, 0, 0);
         }
+}
+
+// O is summed in two levels: kFlushPages pages into registers, which then join
+// the wave's part of the epilogue's LDS (free during a unit's page loop).  The
+// rounding error grows with the square root of the longest chain of additions,
+// and long units are the fast ones (16 rows of 16k to 32k tokens, 64/8 heads,
+// fp16: 358 us a layer in 64-page units, 278 in 512-page ones, whose error
+// against float64 was 4.5e-7 in one level against 2.9e-7, and is 2.8e-7 in two).
+// The registers are all in use, so LDS is the second level.  Whole pairs, which
+// the split size never lengthens, and the general shapes, which the longer loop
+// slows by up to 4%, stay in one level, as do mixed steps (2% there, and their
+// units stay short); a flush every 24 fp16 pages takes 0.5%
+// of a step of 256 rows.  fp32 pages add four times per page, fp16 pages once.
+template <typename KT>
+constexpr int kFlushPages = sizeof(KT) == 4 ? 8 : 24;  // pages of one wave
+
+// o[h][e] of the wave's LDS part takes the lane's O, its own old value (unless
+// `first`) brought from the max m_at to the current one.
+template <int D, typename Rows>
+__device__ __forceinline__ void flush_o(WaveState<D>& st, Rows& o, bool first, float& m_at, int G, int n, int g) {
+    f4 ar = {0.f, 0.f, 0.f, 0.f};
+    if (!first) {
+        const float f = fast_exp2(m_at - st.m);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ar[r] = __shfl(f, 4 * g + r);
+    }
+    m_at = st.m;
+    int at = 4 * g * D + 4 * n;  // formed here (the empty asm), not kept in a register through the page loop
+    asm volatile("" : "+v"(at));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (4 * g + r < G) {
+#pragma unroll
+            for (int c = 0; c < D / 64; ++c) {
+                f4* dst = reinterpret_cast<f4*>(&o[0][0] + at + r * D + 64 * c);
+                f4 v;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = st.o[4 * c + i][r];
+                if (!first) v += *dst * ar[r];
+                *dst = v;
+            }
+        }
+    }
+#pragma unroll
+    for (int b = 0; b < D / 16; ++b) st.o[b] = f4{0.f, 0.f, 0.f, 0.f};
 }
 
 template <int D, typename KT, int MODE>
@@ -590,7 +639,8 @@ __device__ __forceinline__ void load_first_page(PageRegs<D, KT>& pr, const Decod
 // page loop, again with nothing else in flight, and the last split of a pair
 // merges it in that unit's epilogue.  A workgroup's last one or two pieces settle after its
 // final unit.
-template <int D, typename KT, int MODE>
+// TWO_LEVEL: split units flush their sums (flush_o).
+template <int D, typename KT, int MODE, bool TWO_LEVEL = MODE == kExact>
 __device__ __forceinline__ void decode_bins_body(const DecodeArgs& a, EpilogueLds<D, kMaxGroupMfma>& sh, int bx,
                                                  int by) {
 
@@ -663,23 +713,56 @@ __device__ __forceinline__ void decode_bins_body(const DecodeArgs& a, EpilogueLd
 
         // Two page buffers in flight: load page p + kDecodeWaves while computing page p.
         int p = u.page_begin + wave;
-        while (p < u.page_end) {
-            const int pn = p + kDecodeWaves;
-            if (pn < u.page_end && !rb_ready) {
-                const int64_t blk = ld_meta(bt + pn * geo.m);
-                load_tile<D, KT, MODE>(rb, a, kbase, vbase, bt, pn, blk, min(geo.tt, u.ctx - pn * geo.tt), n, g, geo);
+        bool flushed = false;  // the wave's LDS part holds pages already
+        float m_at = 0.f;      // their max
+        if constexpr (TWO_LEVEL) {
+            const bool split = (u.split_info >> 16) > 1;
+            while (p < u.page_end) {
+                const int flush_at = split ? min(p + kFlushPages<KT> * kDecodeWaves, u.page_end) : u.page_end;
+                do {
+                    const int pn = p + kDecodeWaves;
+                    if (pn < u.page_end && !rb_ready) {
+                        const int64_t blk = ld_meta(bt + pn * geo.m);
+                        load_tile<D, KT, MODE>(rb, a, kbase, vbase, bt, pn, blk, min(geo.tt, u.ctx - pn * geo.tt), n, g,
+                                               geo);
+                    }
+                    rb_ready = false;
+                    compute_page<D, KT, MODE>(st, ra, q, min(geo.tt, u.ctx - p * geo.tt), g);
+                    p = pn;
+                    if (pn >= u.page_end) break;
+                    const int pnn = pn + kDecodeWaves;
+                    if (pnn < u.page_end) {
+                        const int64_t blk = ld_meta(bt + pnn * geo.m);
+                        load_tile<D, KT, MODE>(ra, a, kbase, vbase, bt, pnn, blk, min(geo.tt, u.ctx - pnn * geo.tt), n,
+                                               g, geo);
+                    }
+                    compute_page<D, KT, MODE>(st, rb, q, min(geo.tt, u.ctx - pn * geo.tt), g);
+                    p = pnn;
+                } while (p < flush_at);
+                if (p < u.page_end) {
+                    flush_o<D>(st, sh.o[wave], !flushed, m_at, G, n, g);
+                    flushed = true;
+                }
             }
-            rb_ready = false;
-            compute_page<D, KT, MODE>(st, ra, q, min(geo.tt, u.ctx - p * geo.tt), g);
-            if (pn >= u.page_end) break;
-            const int pnn = pn + kDecodeWaves;
-            if (pnn < u.page_end) {
-                const int64_t blk = ld_meta(bt + pnn * geo.m);
-                load_tile<D, KT, MODE>(ra, a, kbase, vbase, bt, pnn, blk, min(geo.tt, u.ctx - pnn * geo.tt), n, g,
-                                       geo);
+        } else {
+            while (p < u.page_end) {
+                const int pn = p + kDecodeWaves;
+                if (pn < u.page_end && !rb_ready) {
+                    const int64_t blk = ld_meta(bt + pn * geo.m);
+                    load_tile<D, KT, MODE>(rb, a, kbase, vbase, bt, pn, blk, min(geo.tt, u.ctx - pn * geo.tt), n, g, geo);
+                }
+                rb_ready = false;
+                compute_page<D, KT, MODE>(st, ra, q, min(geo.tt, u.ctx - p * geo.tt), g);
+                if (pn >= u.page_end) break;
+                const int pnn = pn + kDecodeWaves;
+                if (pnn < u.page_end) {
+                    const int64_t blk = ld_meta(bt + pnn * geo.m);
+                    load_tile<D, KT, MODE>(ra, a, kbase, vbase, bt, pnn, blk, min(geo.tt, u.ctx - pnn * geo.tt), n, g,
+                                           geo);
+                }
+                compute_page<D, KT, MODE>(st, rb, q, min(geo.tt, u.ctx - pn * geo.tt), g);
+                p = pnn;
             }
-            compute_page<D, KT, MODE>(st, rb, q, min(geo.tt, u.ctx - pn * geo.tt), g);
-            p = pnn;
         }
 
         // No page load is outstanding here, so these waits are free: the
@@ -712,14 +795,18 @@ __device__ __forceinline__ void decode_bins_body(const DecodeArgs& a, EpilogueLd
             sh.m[wave][n] = st.m;
             sh.l[wave][n] = st.l;
         }
+        if (TWO_LEVEL && flushed) {
+            flush_o<D>(st, sh.o[wave], false, m_at, G, n, g);
+        } else {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int h = 4 * g + r;
-            if (h < G) {
+            for (int r = 0; r < 4; ++r) {
+                const int h = 4 * g + r;
+                if (h < G) {
 #pragma unroll
-                for (int c = 0; c < D / 64; ++c)
+                    for (int c = 0; c < D / 64; ++c)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) sh.o[wave][h][64 * c + 4 * n + i] = st.o[4 * c + i][r];
+                        for (int i = 0; i < 4; ++i) sh.o[wave][h][64 * c + 4 * n + i] = st.o[4 * c + i][r];
+                }
             }
         }
         if (cnt >= 0 && tid == 0) sh.last = prev == (read_unit(a, cnt).split_info >> 16) - 1;

@@ -1233,7 +1233,7 @@ __global__ __launch_bounds__(kDecodeThreads, 2) void paged_mixed_mfma_kernel(Dec
     const int bx = blockIdx.x;
     const int by = blockIdx.y;
     if (bx < num_bins) {
-        if (by < decode_y) decode_bins_body<D, KT, kExact>(da, sh.d, bx, by);
+        if (by < decode_y) decode_bins_body<D, KT, kExact, false>(da, sh.d, bx, by);
     } else if (by < tile_y) {
         prefill_tile<D, KT, TILES, REC>(pa, sh.p, bx - num_bins, by);
     }

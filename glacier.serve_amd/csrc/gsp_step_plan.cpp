@@ -20,10 +20,9 @@ namespace {
 // last, so split merges finish while other work still streams rather than in
 // the kernel's tail.  Two bins per CU (the decode kernels' occupancy) keep a
 // second workgroup streaming while the first one is in a unit epilogue; one
-// workgroup alone can draw the CU's full share of HBM bandwidth, so the split
-// size is scored per CU.  A unit costs its pages plus a fixed transition; a
-// split piece also pays for publishing its partial and for its share of the
-// merge.
+// workgroup alone can draw the CU's full share of HBM bandwidth, so both are
+// balanced per CU.  There a unit costs its pages plus a fixed transition, and a
+// split piece 3 pages more for publishing its partial.
 constexpr int kDecodeBinsPerCu = 2;
 constexpr int64_t kUnitCostPages = 1;
 constexpr int64_t kSplitCostPages = 3;
@@ -39,10 +38,35 @@ constexpr int64_t kUnderloadPagesPerBin = 4;
 
 int64_t unit_cost(int64_t pages, bool split) { return pages + kUnitCostPages + (split ? kSplitCostPages : 0); }
 
-// Makespan (in pages) of LPT-packing the units that `target` produces from
-// the per-query page counts into `bins` bins.
+// What the split size is scored by, in ns.  A tile of the page stream takes its
+// bytes at a CU's share of the bandwidth (25 bytes/ns), or the latency floor of
+// a tile whose bytes take less.  A split piece costs about 4 us beyond its
+// pages.  The longest merge sits on the step's tail: the merging workgroup loads 8
+// pieces per round for each 256 of the group's outputs, about 2.5 us a round
+// under load (groups of 8 assumed; the group is the caller's at attention time).
+// Fitted to sweeps of 8 to 1024 pages per piece over 13 steps (1 to 64 rows,
+// both page types, head_dim 32 to 128); the sizes it picks measured, against
+// those picked with a flat 3 pages per piece (us a layer): 16 rows of 16k to
+// 32k tokens, 64/8 heads, fp16: 512 pages 278, 64 pages 358; 28/4 heads fp32
+// 64 rows up to 4096: 48 pages 64.4, 32 pages 68.8; one 8192-token row: 32 pages
+// 27.9, 8 pages 33.5; 14/2 heads, 4 rows up to 8192: 24 pages 18.1, 8 pages
+// 20.3.  At worst 42.7 against 41.4 (20 rows, one KV head of width 32).
+constexpr int64_t kCuBytesPerNs = 25;
+constexpr int64_t kTileFloorNs = 400;
+constexpr int64_t kUnitNs = 600;
+constexpr int64_t kSplitNs = 4000;
+constexpr int64_t kMergeRoundNs = 2500;
+constexpr int64_t kMergeRoundPieces = 8;
+
+struct SplitCosts {
+    int64_t tile, unit, split, round;
+};
+
+// Modelled time of the step's decode work cut into pieces of at most `target`
+// tiles: the makespan of LPT-packing the units into `bins` bins, and the longest merge.
 int64_t simulate_split(const std::vector<int32_t>& pages, int32_t heads_kv, int32_t target, int64_t bins,
-                       std::vector<int64_t>& count, std::vector<int64_t>& heap) {
+                       const SplitCosts& cost_of, std::vector<int64_t>& count, std::vector<int64_t>& heap) {
+    int32_t pieces = 1;
     // count[2s] whole pairs of s pages, count[2s + 1] split pieces of s pages.
     count.assign(2 * ((size_t)target + 1), 0);
     int32_t longest = 0;
@@ -50,6 +74,7 @@ int64_t simulate_split(const std::vector<int32_t>& pages, int32_t heads_kv, int3
         const int32_t ns = std::min((P + target - 1) / target, gsp::kMaxSplits);
         const int32_t base = P / ns, extra = P % ns;
         const int sp = ns > 1 ? 1 : 0;
+        pieces = std::max(pieces, ns);
         // Pieces of base + 1 pages exist only when extra > 0, and then base < target.
         if (extra) count[2 * ((size_t)base + 1) + sp] += (int64_t)extra * heads_kv;
         count[2 * (size_t)base + sp] += (int64_t)(ns - extra) * heads_kv;
@@ -58,7 +83,7 @@ int64_t simulate_split(const std::vector<int32_t>& pages, int32_t heads_kv, int3
     heap.clear();
     for (int32_t s = longest; s >= 1; --s) {
         for (int sp = 1; sp >= 0; --sp) {
-            const int64_t cost = unit_cost(s, sp == 1);
+            const int64_t cost = s * cost_of.tile + cost_of.unit + (sp == 1 ? cost_of.split : 0);
             for (int64_t c = count[2 * (size_t)s + sp]; c > 0; --c) {
                 if ((int64_t)heap.size() < bins) {
                     heap.push_back(-cost);  // min-heap through negated loads
@@ -73,7 +98,7 @@ int64_t simulate_split(const std::vector<int32_t>& pages, int32_t heads_kv, int3
     }
     int64_t worst = 0;
     for (int64_t x : heap) worst = std::max(worst, -x);
-    return worst;
+    return pieces > 1 ? worst + cost_of.round * ((pieces + kMergeRoundPieces - 1) / kMergeRoundPieces) : worst;
 }
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
@@ -328,11 +353,21 @@ int StepPlanner::plan(const PlanPool& pool, const gsp_step_desc* desc, const Pla
                     if (tot > 0) query_pages_.push_back((int32_t)((tot + tt - 1) / tt));
                 }
             }
+            // Beside prefill tiles the decode units are not what the step waits for,
+            // and their bins' flat costs in tiles stay.
+            SplitCosts costs{1, kUnitCostPages, kSplitCostPages, 0};
+            if (!any_tiles) {
+                const int64_t elem = pd.kv_dtype == GSP_KV_F32 ? 4 : 2;
+                costs.tile = std::max(kTileFloorNs, tt * (pd.head_dim + pd.v_head_dim) * elem / kCuBytesPerNs);
+                costs.unit = kUnitNs;
+                costs.split = kSplitNs;
+                costs.round = kMergeRoundNs * ((8 * (int64_t)pd.v_head_dim + kDecodeThreads - 1) / kDecodeThreads);
+            }
             int64_t best_cost = INT64_MAX;
             for (int32_t cand : kSplitCandidates) {
                 if (cand < min_target) continue;
                 if (T / cand > 16 * bins_max) continue;  // far too many units to be competitive
-                const int64_t c = simulate_split(query_pages_, H, cand, sim_bins, sim_count_, sim_heap_);
+                const int64_t c = simulate_split(query_pages_, H, cand, sim_bins, costs, sim_count_, sim_heap_);
                 if (c <= best_cost) {  // ties go to the larger split (fewer units)
                     best_cost = c;
                     target = cand;
