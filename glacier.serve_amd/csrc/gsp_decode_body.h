@@ -16,10 +16,10 @@
 //   PV step kk uses token 4g + kk:  A = P[head n][token 4g + kk] (the lane's own r = kk),
 //   B = V[token 4g + kk][e], e = 64c + 4n + i for output block 4c + i
 //   result: lane holds O[head 4g + r][e].
-// fp16 pages run the same contractions on v_mfma_f32_16x16x16f16 from the
-// same registers (one rank-16 step covers d = 16j + 4g + 0..3, or tokens
-// 4g + 0..3): K and V are exact in fp16, Q and P enter as hi + lo fp16 pairs,
-// accumulation is fp32.  So each lane reads 16-byte (8-byte for fp16) pieces
+// fp16 pages run the same contractions on the fp16 matrix cores from the same
+// registers (a rank-16 step covers d = 16j + 4g + 0..3; for P.V one rank-32 step
+// takes tokens 4g + 0..3 against p_hi and p_lo): K and V are exact in fp16, Q
+// and P enter as hi + lo fp16 pairs, accumulation is fp32.  So each lane reads 16-byte (8-byte for fp16) pieces
 // of K rows and V rows straight into MFMA operands; the softmax needs one
 // max-reduction across the four lane groups per page and four exp2 per lane.
 // Page loads are raw buffer loads whose descriptor covers only the page's

@@ -931,7 +931,9 @@ int gsp_matmul_batch(gsp_ctx* ctx, int32_t w_type, const void* w_dev, const floa
                          (int)walign);
     int rc = set_device(ctx);
     if (rc) return rc;
-    if (use_matmul_tile(w_type, in_dim, out_dim, batch)) {
+    bool tile = use_matmul_tile(w_type, in_dim, out_dim, batch);
+    int64_t tile_groups = 0, tile_splits = 0, tile_per = 0;
+    if (tile) {
         // Splits: K ranges of at least 8 chunks, about one workgroup per CU (4096 x
         // 4096 at 100 rows Q4_K, 64 tiles: 47.6 us unsplit, 27.4 in 4 ranges, 31.1 in
         // 8; F32 at 256 rows, 128 tiles: 60 us in 2, 67 in 3, where half the CUs run
@@ -946,6 +948,23 @@ int gsp_matmul_batch(gsp_ctx* ctx, int32_t w_type, const void* w_dev, const floa
         int64_t per = (chunks + splits - 1) / splits;
         per = (per + unit - 1) / unit * unit;
         splits = (chunks + per - 1) / per;
+        tile_groups = groups;
+        tile_splits = splits;
+        tile_per = per;
+        // A product captured before its workspace has grown takes the other forms,
+        // which may need none (F32) or less.
+        const bool grows = (size_t)groups * 64 * in_dim * 2 > ctx->d_mmx_halves || (size_t)splits * batch > ctx->d_mmexp_words ||
+                           (splits > 1 && (size_t)splits * batch * out_dim > ctx->d_mm_floats) ||
+                           (w_type == GSP_WTYPE_Q4_K && (size_t)groups * (in_dim / 256) * 1024 > ctx->d_mmxs_floats);
+        if (grows) {
+            bool capturing = false;
+            rc = is_capturing(ctx->stream, &capturing);
+            if (rc) return rc;
+            tile = !capturing;
+        }
+    }
+    if (tile) {
+        const int64_t groups = tile_groups, splits = tile_splits, per = tile_per;
         gsp::MatmulArgs a{};
         a.w = w_dev;
         a.x = x_dev;

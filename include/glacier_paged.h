@@ -252,11 +252,14 @@ int gsp_rope_write_step_ex(gsp_ctx* ctx, gsp_pool* pool, int32_t layer, int32_t 
  * decoded exactly (to the float32 value its format defines, or to its exact
  * fp16 quant and fp32 scale) and sums are fp32.  Q8_0, Q4_K and Q6_K
  * products with at least 16384 outputs (batch x out_dim) at up to 64 batch
- * rows, or at least 196608 outputs, take x as a scaled fp16 pair on the fp16
- * matrix cores (other products keep x in fp32, as F32 ones always do): each
- * element then carries an absolute error of at most
- * ~2^-22 of its row's largest |x| (~22 significant bits for elements near
- * the row max, fewer for much smaller ones; every finite x stays finite).
+ * rows, or at least 196608 outputs, and F32 products of at least 1.5e9
+ * multiply-adds above 64 rows (4e9 up to 64), take x as a scaled fp16 pair on
+ * the fp16 matrix cores (other products keep x in fp32): each element then
+ * carries an absolute error of at most ~2^-22 of its row's largest |x| (~22
+ * significant bits for elements near the row max, fewer for much smaller ones;
+ * every finite x stays finite).  Those F32 products scale their weights the
+ * same way by each 64 weights of a row, and sum rows with infinities or
+ * magnitudes outside 2^-100 .. 2^100 in plain fp32.
  * Results are the same bit for bit on every call.  in_dim must be a multiple
  * of 64 (256 for the K-quants; GSP_E_UNSUPPORTED otherwise, as for other
  * weight types); the reference's block sums are not needed by these types. */

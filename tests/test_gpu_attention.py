@@ -274,3 +274,29 @@ def test_split_merges_are_bit_reproducible(torch_mod, gsp, ctx, kv_dtype):
                 assert np.array_equal(o, outs[0]), f"split {split}: run {r} differs from run 0"
     finally:
         pool.destroy()
+
+
+@pytest.mark.parametrize("geom", [(28, 4, 128, "f32"), (14, 2, 64, "f32"), (32, 8, 128, "f16"), (14, 2, 64, "f16"),
+                                  (32, 2, 128, "f16")], ids=lambda g: f"{g[0]}q{g[1]}kv_d{g[2]}_{g[3]}")
+@pytest.mark.parametrize("split_pages", [33, 97, 200])
+def test_long_split_units_match_oracle(torch_mod, gsp, ctx, geom, split_pages):
+    """Units long enough that a wave's sums flush once or several times (every 8 fp32 or 24 fp16 pages of a wave),
+    with scores spread enough that the max moves between flushes.  Outputs are averages of V over thousands of
+    tokens (|V| below 6): p and q pairs carry 22 bits (2^-22 of |V|, 1.4e-6), the oracle's and the device's fp32
+    sums of at most 6500 terms 2^-24 each a term at worst (4e-4 of an average below 0.05)."""
+    nh, nkv, d, dt = geom
+    print(f"case long units {geom} split={split_pages}", flush=True)
+    step = workloads.small_step(seed=nh + d + split_pages, rows=3, n_heads=nh, n_kv=nkv, head_dim=d, kv_dtype=dt,
+                                ctx_lo=3200, ctx_hi=6500, total_blocks=1400, max_seq_len=8192)
+    q, k, v = workloads.host_values(step)
+    q = (q * np.float32(2.0)).astype(np.float32)
+    pool, keep = to_device_pool(torch_mod, gsp, ctx, step, k, v)
+    ctx.set_decode_path(PATHS["mfma"])
+    try:
+        got = gpu_step(torch_mod, gsp, ctx, step, q, pool, split_pages=split_pages)
+    finally:
+        ctx.set_decode_path(0)
+    ref = oracle_step(step, q, k, v, threads=threads())
+    pool.destroy()
+    assert not np.isnan(got).any()
+    assert max_err(got, ref) <= 3e-5
