@@ -28,6 +28,20 @@ size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 bool is_oom(hipError_t e) { return e == hipErrorOutOfMemory || e == hipErrorMemoryAllocation; }
 
+// Device buffers of the projection products (gsp_matmul_batch).
+struct MatmulBuffers {
+    float* partials = nullptr;  // sums of the K ranges
+    size_t partials_floats = 0;
+    uint16_t* x = nullptr;  // x as fp16 pairs
+    size_t x_halves = 0;
+    int32_t* exp = nullptr;  // their exponents
+    size_t exp_words = 0;
+    float* sums = nullptr;  // Q4_K: block sums of the scaled x
+    size_t sums_floats = 0;
+    int32_t* counters = nullptr;  // small-batch form: per-tile counters, zero between launches
+    size_t counter_words = 0;
+};
+
 }  // namespace
 
 struct gsp_ctx {
@@ -78,17 +92,14 @@ struct gsp_ctx {
     size_t aux_words = 0;
     int32_t* d_aux = nullptr;
     size_t d_aux_words = 0;
-    // Split-K partials of gsp_matmul_batch, and x as fp16 pairs with row exponents (Q8_0).
-    float* d_mm = nullptr;
-    size_t d_mm_floats = 0;
-    uint16_t* d_mmx = nullptr;
-    size_t d_mmx_halves = 0;
-    int32_t* d_mmexp = nullptr;
-    size_t d_mmexp_words = 0;
-    int32_t* d_mmcnt = nullptr;  // small-batch form: per-tile counters, zero between launches
-    size_t d_mmcnt_words = 0;
-    float* d_mmxs = nullptr;  // small-batch Q4_K: block sums of the scaled x
-    size_t d_mmxs_floats = 0;
+    // Workspaces of gsp_matmul_batch: [0] for eager products, [1] for captured
+    // ones.  A graph keeps the addresses it was captured with, so buffers of [1]
+    // are never freed or replaced under it: one that must grow goes to `retired`
+    // until gsp_shutdown, and each is at least twice the last, so the retired
+    // ones stay below the size of those in use.  Eager products never touch [1]:
+    // a replay on another stream runs beside them.
+    MatmulBuffers mm[2];
+    std::vector<void*> retired;
     hipEvent_t aux_done = nullptr;
     bool aux_pending = false;
 
@@ -275,6 +286,67 @@ int ensure_device(gsp_ctx* ctx, T** buf, size_t* cap, size_t count, bool zero) {
     return GSP_OK;
 }
 
+// What a product needs of its workspace, in elements; 0: not used.
+struct MatmulNeeds {
+    size_t partials = 0, x = 0, exp = 0, sums = 0, counters = 0;
+};
+
+// Grows a buffer of captured products while the stream captures.  The old one
+// is retired: nodes captured earlier hold its address.
+template <typename T>
+int grow_captured(gsp_ctx* ctx, T** buf, size_t* cap, size_t count) {
+    if (count <= *cap) return GSP_OK;
+    const size_t n = std::max(count, *cap * 2);
+    // An allocation touches no stream; the relaxed mode lets it through a capture.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    int rc = check_hip(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode");
+    if (rc) return rc;
+    T* fresh = nullptr;
+    const hipError_t e = hipMalloc(reinterpret_cast<void**>(&fresh), n * sizeof(T));
+    rc = check_hip(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode");
+    if (e != hipSuccess) return check_hip(e, "hipMalloc(captured workspace)");
+    if (*buf) ctx->retired.push_back(*buf);
+    *buf = fresh;
+    *cap = n;
+    return rc;
+}
+
+// The workspace of a product, grown to `need`.  Eager products share one, which
+// follows ensure_device; captured ones another (gsp_ctx::mm).  A capture asks
+// that an eager product has grown the eager workspace as far, GSP_E_STATE
+// otherwise as for every other workspace; `cold_capture` products (F32 without
+// partial sums) may be captured first.  Refusals come before anything is changed.
+int matmul_workspace(gsp_ctx* ctx, const MatmulNeeds& need, bool cold_capture, MatmulBuffers** out) {
+    MatmulBuffers& eager = ctx->mm[0];
+    MatmulBuffers& captured = ctx->mm[1];
+    bool capturing = false;
+    int rc = is_capturing(ctx->stream, &capturing);
+    if (rc) return rc;
+    *out = capturing ? &captured : &eager;
+    if (!capturing || !cold_capture) {
+        rc = ensure_device(ctx, &eager.partials, &eager.partials_floats, need.partials, false);
+        if (!rc) rc = ensure_device(ctx, &eager.x, &eager.x_halves, need.x, false);
+        if (!rc) rc = ensure_device(ctx, &eager.exp, &eager.exp_words, need.exp, false);
+        if (!rc) rc = ensure_device(ctx, &eager.sums, &eager.sums_floats, need.sums, false);
+        if (!rc) rc = ensure_device(ctx, &eager.counters, &eager.counter_words, need.counters, true);
+        if (!rc && need.counters && captured.counter_words < eager.counter_words) {
+            // Captured products' counters must be zero before their first replay, and a
+            // capture cannot clear them: they grow here, with the eager ones.
+            if (captured.counters) ctx->retired.push_back(captured.counters);
+            captured.counters = nullptr;
+            captured.counter_words = 0;
+            rc = ensure_device(ctx, &captured.counters, &captured.counter_words, eager.counter_words, true);
+            if (!rc) rc = check_hip(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+        }
+        if (rc || !capturing) return rc;
+    }
+    rc = grow_captured(ctx, &captured.partials, &captured.partials_floats, need.partials);
+    if (!rc) rc = grow_captured(ctx, &captured.x, &captured.x_halves, need.x);
+    if (!rc) rc = grow_captured(ctx, &captured.exp, &captured.exp_words, need.exp);
+    if (!rc) rc = grow_captured(ctx, &captured.sums, &captured.sums_floats, need.sums);
+    return rc;
+}
+
 int validate_pool_desc(const gsp_pool_desc* d) {
     if (!d) return gsp::fail(GSP_E_INVALID_ARG, "pool descriptor is NULL");
     if (d->total_blocks < 1) return gsp::fail(GSP_E_INVALID_ARG, "totalBlocks must be >= 1 (got %d)", d->total_blocks);
@@ -384,11 +456,14 @@ void gsp_shutdown(gsp_ctx* ctx) {
     }
     if (ctx->aux) (void)hipHostFree(ctx->aux);
     if (ctx->d_aux) (void)hipFree(ctx->d_aux);
-    if (ctx->d_mm) (void)hipFree(ctx->d_mm);
-    if (ctx->d_mmx) (void)hipFree(ctx->d_mmx);
-    if (ctx->d_mmexp) (void)hipFree(ctx->d_mmexp);
-    if (ctx->d_mmcnt) (void)hipFree(ctx->d_mmcnt);
-    if (ctx->d_mmxs) (void)hipFree(ctx->d_mmxs);
+    for (const MatmulBuffers& b : ctx->mm) {
+        if (b.partials) (void)hipFree(b.partials);
+        if (b.x) (void)hipFree(b.x);
+        if (b.exp) (void)hipFree(b.exp);
+        if (b.sums) (void)hipFree(b.sums);
+        if (b.counters) (void)hipFree(b.counters);
+    }
+    for (void* p : ctx->retired) (void)hipFree(p);
     if (ctx->part) (void)hipFree(ctx->part);
     if (ctx->counters) (void)hipFree(ctx->counters);
     if (ctx->d_records) (void)hipFree(ctx->d_records);
@@ -931,9 +1006,9 @@ int gsp_matmul_batch(gsp_ctx* ctx, int32_t w_type, const void* w_dev, const floa
                          (int)walign);
     int rc = set_device(ctx);
     if (rc) return rc;
-    bool tile = use_matmul_tile(w_type, in_dim, out_dim, batch);
-    int64_t tile_groups = 0, tile_splits = 0, tile_per = 0;
-    if (tile) {
+    MatmulNeeds need;
+    MatmulBuffers* ws = nullptr;
+    if (use_matmul_tile(w_type, in_dim, out_dim, batch)) {
         // Splits: K ranges of at least 8 chunks, about one workgroup per CU (4096 x
         // 4096 at 100 rows Q4_K, 64 tiles: 47.6 us unsplit, 27.4 in 4 ranges, 31.1 in
         // 8; F32 at 256 rows, 128 tiles: 60 us in 2, 67 in 3, where half the CUs run
@@ -948,23 +1023,6 @@ int gsp_matmul_batch(gsp_ctx* ctx, int32_t w_type, const void* w_dev, const floa
         int64_t per = (chunks + splits - 1) / splits;
         per = (per + unit - 1) / unit * unit;
         splits = (chunks + per - 1) / per;
-        tile_groups = groups;
-        tile_splits = splits;
-        tile_per = per;
-        // A product captured before its workspace has grown takes the other forms,
-        // which may need none (F32) or less.
-        const bool grows = (size_t)groups * 64 * in_dim * 2 > ctx->d_mmx_halves || (size_t)splits * batch > ctx->d_mmexp_words ||
-                           (splits > 1 && (size_t)splits * batch * out_dim > ctx->d_mm_floats) ||
-                           (w_type == GSP_WTYPE_Q4_K && (size_t)groups * (in_dim / 256) * 1024 > ctx->d_mmxs_floats);
-        if (grows) {
-            bool capturing = false;
-            rc = is_capturing(ctx->stream, &capturing);
-            if (rc) return rc;
-            tile = !capturing;
-        }
-    }
-    if (tile) {
-        const int64_t groups = tile_groups, splits = tile_splits, per = tile_per;
         gsp::MatmulArgs a{};
         a.w = w_dev;
         a.x = x_dev;
@@ -975,16 +1033,16 @@ int gsp_matmul_batch(gsp_ctx* ctx, int32_t w_type, const void* w_dev, const floa
         a.batch = batch;
         a.splits = (int32_t)splits;
         a.chunks_per_split = (int32_t)per;
-        rc = ensure_device(ctx, &ctx->d_mmx, &ctx->d_mmx_halves, (size_t)groups * 64 * in_dim * 2, false);
-        if (!rc) rc = ensure_device(ctx, &ctx->d_mmexp, &ctx->d_mmexp_words, (size_t)splits * batch, false);
-        if (!rc && splits > 1) rc = ensure_device(ctx, &ctx->d_mm, &ctx->d_mm_floats, (size_t)splits * batch * out_dim, false);
-        if (!rc && w_type == GSP_WTYPE_Q4_K)
-            rc = ensure_device(ctx, &ctx->d_mmxs, &ctx->d_mmxs_floats, (size_t)groups * (in_dim / 256) * 1024, false);
+        need.x = (size_t)groups * 64 * in_dim * 2;
+        need.exp = (size_t)splits * batch;
+        if (splits > 1) need.partials = (size_t)splits * batch * out_dim;
+        if (w_type == GSP_WTYPE_Q4_K) need.sums = (size_t)groups * (in_dim / 256) * 1024;
+        rc = matmul_workspace(ctx, need, w_type == GSP_WTYPE_F32 && splits == 1, &ws);
         if (rc) return rc;
-        a.xh = ctx->d_mmx;
-        a.xexp = ctx->d_mmexp;
-        a.split_out = splits > 1 ? ctx->d_mm : nullptr;
-        a.xsum = w_type == GSP_WTYPE_Q4_K ? ctx->d_mmxs : nullptr;
+        a.xh = ws->x;
+        a.xexp = ws->exp;
+        a.split_out = splits > 1 ? ws->partials : nullptr;
+        a.xsum = w_type == GSP_WTYPE_Q4_K ? ws->sums : nullptr;
         return check_hip(gsp::launch_matmul_tile(a, ctx->stream), "matmul launch");
     }
     if ((w_type == GSP_WTYPE_Q8_0 || w_type == GSP_WTYPE_Q4_K || w_type == GSP_WTYPE_Q6_K) && batch <= 64 &&
@@ -1030,19 +1088,21 @@ int gsp_matmul_batch(gsp_ctx* ctx, int32_t w_type, const void* w_dev, const floa
         a.batch = batch;
         a.splits = (int32_t)splits;
         a.chunks_per_split = (int32_t)per;
-        rc = ensure_device(ctx, &ctx->d_mmx, &ctx->d_mmx_halves, (size_t)gsp::matmul_small_x_halves(batch, in_dim), false);
-        if (!rc) rc = ensure_device(ctx, &ctx->d_mmexp, &ctx->d_mmexp_words, (size_t)splits * batch, false);
-        if (!rc && splits > 1) rc = ensure_device(ctx, &ctx->d_mm, &ctx->d_mm_floats, (size_t)splits * batch * tiles * 64, false);
-        if (!rc && splits > 1) rc = ensure_device(ctx, &ctx->d_mmcnt, &ctx->d_mmcnt_words, (size_t)tiles, true);
-        if (!rc && w_type == GSP_WTYPE_Q4_K)
-            rc = ensure_device(ctx, &ctx->d_mmxs, &ctx->d_mmxs_floats, (size_t)splits * 2 * per * 64, false);
+        need.x = (size_t)gsp::matmul_small_x_halves(batch, in_dim);
+        need.exp = (size_t)splits * batch;
+        if (splits > 1) {
+            need.partials = (size_t)splits * batch * tiles * 64;
+            need.counters = (size_t)tiles;
+        }
+        if (w_type == GSP_WTYPE_Q4_K) need.sums = (size_t)splits * 2 * per * 64;
+        rc = matmul_workspace(ctx, need, false, &ws);
         if (rc) return rc;
-        a.xh = ctx->d_mmx;  // x in tile order, both halves
-        a.xl = ctx->d_mmx;
-        a.xexp = ctx->d_mmexp;
-        a.split_out = splits > 1 ? ctx->d_mm : nullptr;
-        a.counters = splits > 1 ? ctx->d_mmcnt : nullptr;
-        a.xsum = w_type == GSP_WTYPE_Q4_K ? ctx->d_mmxs : nullptr;
+        a.xh = ws->x;  // x in tile order, both halves
+        a.xl = ws->x;
+        a.xexp = ws->exp;
+        a.split_out = splits > 1 ? ws->partials : nullptr;
+        a.counters = splits > 1 ? ws->counters : nullptr;
+        a.xsum = w_type == GSP_WTYPE_Q4_K ? ws->sums : nullptr;
         return check_hip(gsp::launch_matmul_small(a, ctx->stream), "matmul launch");
     }
     // Split K over grid.z until the grid has about two workgroups (64 weight rows
@@ -1069,26 +1129,27 @@ int gsp_matmul_batch(gsp_ctx* ctx, int32_t w_type, const void* w_dev, const floa
     a.xh = nullptr;
     a.xl = nullptr;
     a.xexp = nullptr;
-    if ((w_type == GSP_WTYPE_Q8_0 || w_type == GSP_WTYPE_Q4_K || w_type == GSP_WTYPE_Q6_K) &&
-        (int64_t)batch * out_dim >= kMatmulF16MinOutputs) {
+    const bool f16 = w_type != GSP_WTYPE_F32 && (int64_t)batch * out_dim >= kMatmulF16MinOutputs;
+    const size_t halves = (size_t)batch * in_dim;
+    if (f16) {
         // Large Q8_0 and K-quant products run on the fp16 matrix cores with x as
         // scaled fp16 pairs (Q4_K also with x's block sums for its min term);
         // below the threshold the pre-pass launch costs more than it saves.
-        const size_t halves = (size_t)batch * in_dim;
-        rc = ensure_device(ctx, &ctx->d_mmx, &ctx->d_mmx_halves, 2 * halves, false);
-        if (!rc) rc = ensure_device(ctx, &ctx->d_mmexp, &ctx->d_mmexp_words, (size_t)batch, false);
-        if (!rc && w_type == GSP_WTYPE_Q4_K)
-            rc = ensure_device(ctx, &ctx->d_mmxs, &ctx->d_mmxs_floats, (size_t)batch * (in_dim / 32), false);
-        if (rc) return rc;
-        a.xh = ctx->d_mmx;
-        a.xl = ctx->d_mmx + halves;
-        a.xexp = ctx->d_mmexp;
-        a.xsum = w_type == GSP_WTYPE_Q4_K ? ctx->d_mmxs : nullptr;
+        need.x = 2 * halves;
+        need.exp = (size_t)batch;
+        if (w_type == GSP_WTYPE_Q4_K) need.sums = (size_t)batch * (in_dim / 32);
     }
-    if (splits > 1) {
-        rc = ensure_device(ctx, &ctx->d_mm, &ctx->d_mm_floats, (size_t)splits * batch * out_dim, false);
+    if (splits > 1) need.partials = (size_t)splits * batch * out_dim;
+    if (f16 || splits > 1) {
+        rc = matmul_workspace(ctx, need, false, &ws);
         if (rc) return rc;
-        a.split_out = ctx->d_mm;
+        if (f16) {
+            a.xh = ws->x;
+            a.xl = ws->x + halves;
+            a.xexp = ws->exp;
+            a.xsum = w_type == GSP_WTYPE_Q4_K ? ws->sums : nullptr;
+        }
+        if (splits > 1) a.split_out = ws->partials;
     }
     return check_hip(gsp::launch_matmul(a, ctx->stream), "matmul launch");
 }

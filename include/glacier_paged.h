@@ -260,7 +260,15 @@ int gsp_rope_write_step_ex(gsp_ctx* ctx, gsp_pool* pool, int32_t layer, int32_t 
  * every finite x stays finite).  Those F32 products scale their weights the
  * same way by each 64 weights of a row, and sum rows with infinities or
  * magnitudes outside 2^-100 .. 2^100 in plain fp32.
- * Results are the same bit for bit on every call.  in_dim must be a multiple
+ * Results are the same bit for bit on every call, captured or not.
+ * Graph capture: run the product, or a larger one of its kind, once before
+ * capturing it (a capture that finds the workspace too small fails with
+ * GSP_E_STATE and enqueues nothing; F32 products whose K is not split need no
+ * such call).  Captured products use buffers of their own, which eager calls
+ * never touch and which stay until gsp_shutdown: their graphs stay valid
+ * whatever is called afterwards, and may run beside eager products.  The
+ * captured products of a context share those buffers, so their graphs must
+ * not run at the same time as each other.  in_dim must be a multiple
  * of 64 (256 for the K-quants; GSP_E_UNSUPPORTED otherwise, as for other
  * weight types); the reference's block sums are not needed by these types. */
 int gsp_matmul_batch(gsp_ctx* ctx, int32_t w_type, const void* w_dev, const float* x_dev, float* y_dev,

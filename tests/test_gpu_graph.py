@@ -275,3 +275,110 @@ def test_captured_projection_replays_match_eager(torch_mod, gsp, ctx, w_type, sh
         del graph
     finally:
         ctx.set_stream(None)
+
+
+def _capture_product(torch, ctx, stream, w_type, wd, xd, shape):
+    """(graph, output) of one captured gsp_matmul_batch."""
+    in_dim, out_dim, batch = shape
+    out = torch.full((batch, out_dim), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=stream):
+        ctx.matmul_batch(w_type, wd.data_ptr(), xd.data_ptr(), out.data_ptr(), in_dim, out_dim, batch)
+    assert set(_graph_node_types(graph)) == {HIP_GRAPH_NODE_KERNEL}
+    graph.instantiate()
+    return graph, out
+
+
+# Products of the tile form (unsplit F32, Q4_K in K ranges) and of the small-batch form.
+CAPTURED = [(0, (1024, 8192, 256)), (12, (2048, 2100, 350)), (8, (3584, 3584, 64))]
+
+
+def test_captured_projections_survive_larger_eager_products(torch_mod, gsp):
+    """Graphs of projections keep their buffers: larger eager products grow the context's workspace
+    after the captures, every replay still matches the eager product bit for bit, and a second
+    capture that needs larger buffers leaves the earlier graphs theirs."""
+    torch = torch_mod
+    rng = np.random.default_rng(77)
+    stream = torch.cuda.Stream()
+    with gsp.Context(0) as fresh:
+        fresh.set_stream(stream.cuda_stream)
+
+        def operands(w_type, shape):
+            in_dim, out_dim, batch = shape
+            if w_type == 0:
+                wd = torch.from_numpy(rng.standard_normal((out_dim, in_dim)).astype(np.float32)).cuda()
+            else:
+                wd = torch.from_numpy(_raw_weights(rng, w_type, out_dim, in_dim)).cuda()
+            return wd, torch.from_numpy(rng.standard_normal((batch, in_dim)).astype(np.float32)).cuda()
+
+        def eager(w_type, wd, xd, shape):
+            y = torch.full((shape[2], shape[1]), float("nan"), device="cuda")
+            torch.cuda.synchronize()
+            fresh.matmul_batch(w_type, wd.data_ptr(), xd.data_ptr(), y.data_ptr(), *shape)
+            fresh.sync()
+            return y
+
+        cases = []
+        for w_type, shape in CAPTURED:
+            wd, xd = operands(w_type, shape)
+            want = eager(w_type, wd, xd, shape)
+            cases.append((w_type, shape, wd, xd, want) + _capture_product(torch, fresh, stream, w_type, wd, xd, shape))
+        # Larger products of the same kinds: eager, then captured too.
+        larger = [(0, (2048, 8192, 520)), (12, (4096, 4100, 700)), (8, (3584, 9000, 64))]
+        for w_type, shape in larger:
+            wd, xd = operands(w_type, shape)
+            want = eager(w_type, wd, xd, shape)
+            cases.append((w_type, shape, wd, xd, want) + _capture_product(torch, fresh, stream, w_type, wd, xd, shape))
+        for rep in range(3):
+            for w_type, shape, wd, xd, want, graph, out in cases:
+                print(f"replay {rep} type={w_type} {shape}", flush=True)
+                out.fill_(float("nan"))
+                torch.cuda.synchronize()
+                graph.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(out, want), f"replay {rep} of {w_type} {shape}"
+                assert torch.equal(eager(w_type, wd, xd, shape), want)
+        cases.clear()
+        fresh.set_stream(None)
+
+
+@pytest.mark.filterwarnings("ignore:The CUDA Graph is empty")
+def test_first_capture_of_a_projection(torch_mod, gsp):
+    """On a context with no workspace an unsplit F32 product can be captured and takes the form the
+    eager call takes (equal bit for bit); a product that needs partial sums, and a quantized one, are
+    refused and leave the context usable."""
+    torch = torch_mod
+    rng = np.random.default_rng(78)
+    stream = torch.cuda.Stream()
+    with gsp.Context(0) as fresh:
+        fresh.set_stream(stream.cuda_stream)
+        shape = (1024, 8192, 256)
+        wd = torch.from_numpy(rng.standard_normal((8192, 1024)).astype(np.float32)).cuda()
+        xd = torch.from_numpy(rng.standard_normal((256, 1024)).astype(np.float32)).cuda()
+        graph, out = _capture_product(torch, fresh, stream, 0, wd, xd, shape)
+        q_shape = (2048, 2100, 350)
+        qd = torch.from_numpy(_raw_weights(rng, 12, 2100, 2048)).cuda()
+        qx = torch.from_numpy(rng.standard_normal((350, 2048)).astype(np.float32)).cuda()
+        y = torch.empty((350, 2100), device="cuda")
+        torch.cuda.synchronize()
+        refused = torch.cuda.CUDAGraph()
+        with pytest.raises(gsp.StateError, match="capturing"):
+            with torch.cuda.graph(refused, stream=stream):
+                fresh.matmul_batch(12, qd.data_ptr(), qx.data_ptr(), y.data_ptr(), *q_shape)
+        del refused
+        want = torch.full((256, 8192), float("nan"), device="cuda")
+        torch.cuda.synchronize()
+        fresh.matmul_batch(0, wd.data_ptr(), xd.data_ptr(), want.data_ptr(), *shape)
+        fresh.sync()
+        for rep in range(3):
+            out.fill_(float("nan"))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), f"replay {rep}"
+            fresh.matmul_batch(12, qd.data_ptr(), qx.data_ptr(), y.data_ptr(), *q_shape)
+            fresh.sync()
+            assert torch.isfinite(y).all()
+        del graph
+        fresh.set_stream(None)
