@@ -959,8 +959,9 @@ constexpr int64_t kMatmulSmallMinOutputs = 16384;
 //   Q4_K above 64 rows: 4096 x 4096 at 1024 185 -> 102, at 100 34.7 -> 28.9,
 //     4096 x 16384 at 65 76 -> 52, 1024 x 1024 at 3000 46 -> 42; below the line
 //     3584 x 3584 at 65 27.6 -> 27.6, 3584 x 512 at 2048 59 -> 64.
-//   Q4_K up to 64 rows, by the weights alone: 4096 x 32768 at 16 68 -> 31, 3584
-//     x 18944 at 64 58 -> 46, 4096 x 8192 at 33 29.7 -> 28.2; below 4096 x 6144 at 48 27.1 -> 27.8,
+//   Q4_K up to 64 rows, by the weights alone: 4096 x 32768 at 1 60.7 -> 28.8, at
+//     15 67 -> 30, 3584 x 18944 at 4 40.5 -> 24.3, at 64 58 -> 46, 4096 x 8192 at
+//     15 23.1 -> 16.8, at 33 29.7 -> 28.2; below 4096 x 6144 at 48 27.1 -> 27.8,
 //     4096 x 4096 at 64 21.8 -> 24.3.
 //   Q8_0 above 64 rows: 4096 x 4096 at 1024 177 -> 113, 3584 x 3584 at 300 56
 //     -> 51; below 128 rows 30.5 -> 32.1.  Up to 64 rows only the widest outputs
@@ -971,6 +972,8 @@ constexpr int64_t kMatmulSmallMinOutputs = 16384;
 //     46.5 -> 41.3, 18944 x 3584 at 64 114 -> 96; below 4096 x 1024 at 300 37.8
 //     -> 39.7, 4096 x 16384 at 33 76 -> 79.
 static bool use_matmul_tile(int32_t w_type, int64_t in_dim, int64_t out_dim, int64_t batch) {
+    // Quantized products with fewer outputs than the header states keep x in fp32.
+    if (w_type != GSP_WTYPE_F32 && batch * out_dim < (batch > 64 ? kMatmulF16MinOutputs : kMatmulSmallMinOutputs)) return false;
     // The kernel's 32-row descriptors and its workgroup index are 32-bit.
     if (in_dim * 4 * 32 > INT32_MAX || (out_dim + 127) / 128 * ((batch + 63) / 64) > INT32_MAX / 64) return false;
     const double macs = (double)batch * (double)in_dim * (double)out_dim;

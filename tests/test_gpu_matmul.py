@@ -332,3 +332,42 @@ def test_tile_form_f32_beyond_the_fp16_pairs(torch_mod, gsp, ctx):
     # fp32 sums of K terms round to 1e-5 of the terms' magnitude at worst; rows of 1e-37 lose their
     # products below the smallest normal (K terms of half 2^-149 each, and flushed subnormals of 2^-126).
     assert np.all(np.abs(got[kinds] - ref[kinds]) <= 1e-5 * mag[kinds] + in_dim * 2.0 ** -126)
+
+
+# Products whose weights would suit the tile form but whose outputs are too few for x as fp16 pairs
+# (the header's line: 16384 outputs up to 64 rows, 196608 above): x stays in fp32.
+FEW_OUTPUTS = [
+    (orc.WTYPE_Q4_K, 4096, 8200, 1),
+    (orc.WTYPE_Q4_K, 14848, 1024, 100),
+    (orc.WTYPE_Q8_0, 24576, 2048, 65),
+    (orc.WTYPE_Q6_K, 26368, 2048, 65),
+]
+
+
+@pytest.mark.parametrize("w_type,in_dim,out_dim,batch", FEW_OUTPUTS, ids=lambda v: str(v))
+def test_products_with_few_outputs_keep_x_in_fp32(torch_mod, gsp, ctx, w_type, in_dim, out_dim, batch):
+    """One channel of every row is 1e12 times the rest and meets only zero weights (its blocks' scales
+    are zero).  With x in fp32 the other channels keep their bits and the fp32 summation bar holds; a
+    pair scaled to the row's largest value would carry 3e-12 of it (2^-38), far above the bar."""
+    print(f"case matmul few outputs type={w_type} {in_dim}x{out_dim} b{batch}", flush=True)
+    rng = np.random.default_rng(in_dim + out_dim + batch + w_type)
+    if w_type == orc.WTYPE_Q8_0:
+        data, wm = _weights(rng, w_type, out_dim, in_dim)
+        data, block, scales, decode = np.array(data), (in_dim // 32, 34), (slice(0, 2),), orc.q8_0_decode
+    else:
+        data, wm = _kquant_weights(rng, w_type, out_dim, in_dim)
+        data = np.array(data)
+        q4 = w_type == orc.WTYPE_Q4_K
+        block = (in_dim // orc.QK_K, orc.Q4_K_BYTES if q4 else orc.Q6_K_BYTES)
+        scales = (slice(0, 4),) if q4 else (slice(208, 210),)
+        decode = orc.q4_k_decode if q4 else orc.q6_k_decode
+    for s in scales:
+        data.view(np.uint8).reshape(out_dim, *block)[:, 1, s] = 0
+    wm = np.asarray(decode(data, out_dim, in_dim), np.float64)
+    loud = (32 if w_type == orc.WTYPE_Q8_0 else 256) + 5
+    assert not wm[:, loud].any() and wm[:, 0].any()
+    x = rng.standard_normal((batch, in_dim)).astype(np.float32)
+    x[:, loud] *= np.float32(1e12)
+    got = _run(torch_mod, gsp, ctx, w_type, data, x, in_dim, out_dim)
+    x64 = x.astype(np.float64)
+    assert np.all(np.abs(got - x64 @ wm.T) <= 1e-5 * (np.abs(x64) @ np.abs(wm).T) + 1e-7)
