@@ -1309,8 +1309,9 @@ __global__ __launch_bounds__(kMmThreads, 2) void matmul_q6k_f16_small_kernel(Mat
 //   Q4_K: lane group g owns quarter g of the super-block (sub-blocks 2 g and
 //     2 g + 1, 32 contiguous quant bytes).  sc * (q - 8) is exact in fp16, so
 //     only d remains outside, one fma per chunk.  The min term dmin m - 8 d sc
-//     is two matrix steps per super-block: the 8 sub-block sums of x as fp16
-//     pairs (from the pre-pass, times 2^-6) against the 6-bit mins and scales.
+//     is two matrix steps per super-block: the 8 sub-block sums of x, each in
+//     three halves that hold its fp32 value (from the pre-pass, times 2^-6),
+//     against the 6-bit mins and scales.
 //   Q6_K: lane group g owns l = 16 (g % 2) .. + 15 of each quarter of half
 //     g / 2.  m = sc * (q - 32), at most 4096, takes two halves: its fp16
 //     rounding and the rest (0 or +-1), three matrix steps instead of the four
@@ -1352,6 +1353,9 @@ struct KOrder {
 constexpr int kXPlain = 1 << 16;
 constexpr int kTileHalves = 2048;   // one M tile of a chunk: [block][hi, lo][lane][8 halves]
 constexpr int kXBlockSumLog2 = 6;   // Q4_K's sub-block sums of x enter times 2^-6 (32 values below 2^13 each)
+// The second and third halves of a sum are stored over these factors, which the
+// weights' side carries (6-bit values times them are exact, normal halves).
+constexpr float kSumScale1 = 1.0f / (1 << 11), kSumScale2 = 1.0f / (1 << 14);
 
 // x of batch row b over K range z as scaled fp16 pairs in tile order,
 // [64-row group][chunk][M tile][block][hi, lo][lane g * 16 + m][8 halves], with
@@ -1432,20 +1436,22 @@ __global__ __launch_bounds__(kMmThreads) void matmul_split_x_tile_kernel(MatmulA
             *reinterpret_cast<h8*>(dst + (g * 16 + m) * 8 + 512) = lo;
         }
         if constexpr (WT == kWeightQ4_K) {
-            // Four consecutive threads hold a sub-block's 32 values.  Its sum is a pair of
-            // halves in the lane group's slot 2 * (sub-block % 2) of the row's sums operand,
-            // [64-row group][super-block][M tile][lane][8 halves], the upper four halves zero.
+            // Four consecutive threads hold a sub-block's 32 values.  Its fp32 sum is three
+            // halves (11 + 11 + 2 bits, so all of it) in the lane group's slot 4 * (sub-block % 2)
+            // of the row's sums operand, [64-row group][super-block][M tile][lane][8 halves].
             sm += __shfl_xor(sm, 1);
             sm += __shfl_xor(sm, 2);
             if ((i & 3) == 0) {
                 const float v = sm * (1.0f / (1 << kXBlockSumLog2));
-                const _Float16 vh = (_Float16)v;
-                const _Float16 vl = (_Float16)(__builtin_isinf(v) ? 0.f : v - (float)vh);
+                const bool inf = __builtin_isinf(v);  // rides on its first half alone
+                const _Float16 v0 = (_Float16)v;
+                const float r1 = inf ? 0.f : (v - (float)v0) * (1.0f / kSumScale1);
+                const _Float16 v1 = (_Float16)r1;
+                const _Float16 v2 = (_Float16)((r1 - (float)v1) * (kSumScale1 / kSumScale2));
                 const int sub = (k >> 5) & 7;
                 _Float16* sd = reinterpret_cast<_Float16*>(a.xsum) +
                                (((row0 >> 2) + (k >> 8)) * 4 + tile) * 512 + ((sub >> 1) * 16 + m) * 8;
-                *reinterpret_cast<h2*>(sd + 2 * (sub & 1)) = h2{vh, vl};
-                *reinterpret_cast<h2*>(sd + 4 + 2 * (sub & 1)) = h2{(_Float16)0.f, (_Float16)0.f};
+                *reinterpret_cast<h4v*>(sd + 4 * (sub & 1)) = h4v{v0, v1, v2, (_Float16)0.f};
             }
         }
     };
@@ -1479,6 +1485,13 @@ typedef uint32_t u2v __attribute__((ext_vector_type(2)));
 typedef uint32_t u3v __attribute__((ext_vector_type(3)));
 
 __device__ __forceinline__ h2 splat2(_Float16 v) { return h2{v, v}; }
+
+// The weights' side of Q4_K's sums operand: the 6-bit values of two sub-blocks against three halves each.
+__device__ __forceinline__ h8 sums_operand(h2 q) {
+    const h2 q1 = q * splat2((_Float16)kSumScale1);
+    const h2 q2 = q * splat2((_Float16)kSumScale2);
+    return h8{q[0], q1[0], q2[0], 0, q[1], q1[1], q2[1], 0};
+}
 
 template <int WT>
 struct TileW;
@@ -1908,8 +1921,8 @@ __device__ __forceinline__ void tile_products(const MatmulArgs& a, TileW<WT>& w,
             if constexpr (CC == 0) {  // the super-block's min term, dmin m - 8 d sc against the sums of x
 #pragma unroll
                 for (int j = 0; j < NT; ++j) {
-                    const h8 mb = h8{w.mp[j][0], w.mp[j][0], w.mp[j][1], w.mp[j][1], 0, 0, 0, 0};
-                    const h8 sb = h8{w.sp[j][0], w.sp[j][0], w.sp[j][1], w.sp[j][1], 0, 0, 0, 0};
+                    const h8 mb = sums_operand(w.mp[j]);
+                    const h8 sb = sums_operand(w.sp[j]);
                     const float d8 = w.d[j] * (float)(8 << kXBlockSumLog2);
 #pragma unroll
                     for (int t = 0; t < MT; ++t) {

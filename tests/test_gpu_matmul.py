@@ -371,3 +371,29 @@ def test_products_with_few_outputs_keep_x_in_fp32(torch_mod, gsp, ctx, w_type, i
     got = _run(torch_mod, gsp, ctx, w_type, data, x, in_dim, out_dim)
     x64 = x.astype(np.float64)
     assert np.all(np.abs(got - x64 @ wm.T) <= 1e-5 * (np.abs(x64) @ np.abs(wm).T) + 1e-7)
+
+
+def test_tile_form_q4_k_min_term_keeps_the_fp32_sums(torch_mod, gsp, ctx):
+    """Weights that are all -1 (d = 0, dmin = 1, mins 1): y = -sum x.  Two sub-blocks of a super-block hold
+    integers whose sums, near +2^23.5 and -2^23.5, need all 24 bits; every partial sum is an integer of at
+    most 2^24, so fp32 gives the sum of x exactly, and fewer bits of the sub-block sums would not."""
+    in_dim, out_dim, batch = 4096, 8200, 70
+    rng = np.random.default_rng(24)
+    b = np.zeros((out_dim, in_dim // orc.QK_K, orc.Q4_K_BYTES), np.uint8)
+    b[..., 2:4] = np.array([1.0], np.float16).view(np.uint8)
+    b[..., 8:12] = 1    # mins of sub-blocks 0..3, and their low bits of 4..7
+    b[..., 12:16] = 0x10  # mins of sub-blocks 4..7
+    data = b.reshape(-1)
+    assert np.all(orc.q4_k_decode(data[: in_dim // orc.QK_K * orc.Q4_K_BYTES], 1, in_dim) == -1.0)
+    x = np.zeros((batch, in_dim // 32, 32), np.float32)
+    for row in range(batch):
+        pair = 2 * rng.integers(0, in_dim // 64)
+        a = rng.integers(330000, 400000, 32)
+        c = rng.integers(330000, 400000, 32)
+        a[0] += 1 - int(a.sum()) % 2  # odd sums
+        c[0] += 1 - int(c.sum()) % 2
+        x[row, pair], x[row, pair + 1] = a, -c
+    x = x.reshape(batch, in_dim)
+    assert np.all(np.abs(x.reshape(batch, -1, 32).sum(-1, dtype=np.float64)).max(-1) > 2.0 ** 23)
+    got = _run(torch_mod, gsp, ctx, orc.WTYPE_Q4_K, data, x, in_dim, out_dim)
+    assert np.array_equal(got, np.repeat(-x.sum(-1, dtype=np.float64)[:, None], out_dim, 1))
