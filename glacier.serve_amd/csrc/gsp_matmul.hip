@@ -1909,6 +1909,7 @@ __device__ __forceinline__ void tile_products(const MatmulArgs& a, TileW<WT>& w,
         constexpr int S = decltype(s_t)::value;
         constexpr int CC = S % kUnit;
         stage_x(std::integral_constant<int, (S + 3) % 4>{}, c + 3);
+        __builtin_amdgcn_sched_barrier(0x78F);  // no vector memory access crosses: kLater counts the fetches below as later
         if constexpr (WT == kWeightF32) {
             w.template expand<CC>(S % 2);
             w.fetch(S % 2, min(c + 2, c_end - 1));
