@@ -1292,7 +1292,7 @@ __global__ __launch_bounds__(kMmThreads, 2) void matmul_q6k_f16_small_kernel(Mat
 // staged in LDS serves all four waves and two N tiles, and a wave expands its
 // own rows' words to fp16 operands in registers once per chunk of 64 k and uses
 // each for four M tiles.  Measured at 1024 rows of 4096 x 4096 (us): Q8_0 177 ->
-// 113, Q4_K 185 -> 102, Q6_K 194 -> 136, F32 279 -> 166, about 700 TFLOP/s of
+// 107, Q4_K 185 -> 101, Q6_K 194 -> 136, F32 279 -> 173, about 700 TFLOP/s of
 // fp16 matrix steps; what is left is instruction issue (a chunk of Q6_K is
 // 48 matrix steps and 130 vector instructions a wave; dropping the expansion
 // or the scaling takes it to 128 us each, the barriers nothing).
@@ -1319,11 +1319,14 @@ __global__ __launch_bounds__(kMmThreads, 2) void matmul_q6k_f16_small_kernel(Mat
 //   F32: as Q8_0, but a lane's eight values are k = 32 blk + 4 g .. + 3 and 16
 //     further on, so that one load instruction covers 64 contiguous bytes of
 //     each row.  They enter as an fp16 pair scaled by the row's largest |w| of
-//     the chunk (2^e, applied with the chunk's sum); as for x, the pair keeps all
-//     but ~2^-24 of the element, and the lo x lo product (at most 2^-24,
-//     typically 2^-27 of the term) is left out.  Against float64 the products
-//     are closer than the fp32 form's (4096 x 4096 at 256 rows: 8.4e-7 ->
-//     1.5e-7): a running sum rounds once a chunk instead of once per four k.
+//     the chunk (2^e, applied with the chunk's sum).  A pair keeps 22 bits of an
+//     element, or 2^-38 of the scale's largest where that is more, and the lo x
+//     lo product (at most 2^-22, typically 2^-25 of the term) is left out;
+//     operands whose range is too wide for that, or that leave fp16's, go to
+//     plain_products (kWideLog2, kXPlain; the check costs 4 of 62 us at 256
+//     rows).  Against float64 the products are closer than the fp32 form's
+//     (4096 x 4096 at 256 rows: 8.4e-7 -> 1.6e-7): a running sum rounds once a
+//     chunk instead of once per four k.
 // K is split over ranges only where the tiles leave CUs idle; the ranges' sums
 // are then added in order by matmul_reduce_kernel.
 template <int WT>
@@ -1348,9 +1351,20 @@ struct KOrder {
 };
 
 // Added to a row's exponent when the fp16 pairs cannot stand for the row (F32
-// products: an infinite element, or a row whose largest |x| is below 2^-113):
-// its outputs are summed in plain fp32 instead.
+// products: an infinite element, a row whose largest |x| is below 2^-113, or one
+// of a wide range): its outputs are summed in plain fp32 instead.
 constexpr int kXPlain = 1 << 16;
+// A scaled pair holds an element to 2^-23 of itself or 2^-38 of the scale's
+// largest, whichever is more (the matrix cores keep fp16 subnormals).  F32
+// operands are wide, and summed in plain fp32, when four neighbours lie below
+// 2^-kWideLog2 of the largest and are not all zero: every group of four then
+// keeps 22 bits of its own largest.  (Among 4096 normal values beside a channel
+// 12 times as loud that happens once in 10^9 rows.)
+constexpr int kWideLog2 = 16;
+// `low`: the least, over the groups, of the bits of a group's largest magnitude minus one (zero groups wrap to the top).
+__device__ __forceinline__ bool wide_row(uint32_t low, float mx) {
+    return low + 1 < __float_as_uint(mx * (1.0f / (1 << kWideLog2))) && low != ~0u;
+}
 constexpr int kTileHalves = 2048;   // one M tile of a chunk: [block][hi, lo][lane][8 halves]
 constexpr int kXBlockSumLog2 = 6;   // Q4_K's sub-block sums of x enter times 2^-6 (32 values below 2^13 each)
 // The second and third halves of a sum are stored over these factors, which the
@@ -1363,6 +1377,7 @@ constexpr float kSumScale1 = 1.0f / (1 << 11), kSumScale2 = 1.0f / (1 << 14);
 template <int WT>
 __global__ __launch_bounds__(kMmThreads) void matmul_split_x_tile_kernel(MatmulArgs a) {
     __shared__ float red[kMmThreads / 64];
+    __shared__ uint32_t red_low[kMmThreads / 64];
     const int b = blockIdx.x;
     const int z = blockIdx.y;
     const int t = threadIdx.x;
@@ -1374,10 +1389,12 @@ __global__ __launch_bounds__(kMmThreads) void matmul_split_x_tile_kernel(MatmulA
     const bool held = np <= kHeld * kMmThreads;
     f4 hv[kHeld][2];
     float mx = 0.f;
+    uint32_t low = ~0u;  // F32: see kWideRow
     auto max8 = [&](const f4& u, const f4& v) {
         const float mu = fmaxf(fmaxf(fabsf(u[0]), fabsf(u[1])), fmaxf(fabsf(u[2]), fabsf(u[3])));
         const float mv = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
         mx = fmaxf(mx, fmaxf(mu, mv));
+        if constexpr (WT == kWeightF32) low = min(low, min(__float_as_uint(mu) - 1, __float_as_uint(mv) - 1));
     };
     if (held) {
 #pragma unroll
@@ -1397,6 +1414,11 @@ __global__ __launch_bounds__(kMmThreads) void matmul_split_x_tile_kernel(MatmulA
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
     if ((t & 63) == 0) red[t >> 6] = mx;
+    if constexpr (WT == kWeightF32) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) low = min(low, (uint32_t)__shfl_xor((int)low, off));
+        if ((t & 63) == 0) red_low[t >> 6] = low;
+    }
     __syncthreads();
     mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     int ex = 0;
@@ -1465,7 +1487,9 @@ __global__ __launch_bounds__(kMmThreads) void matmul_split_x_tile_kernel(MatmulA
         for (int i = t; i < np; i += kMmThreads) put(i, xr[2 * i], xr[2 * i + 1]);
     }
     if (t == 0) {
-        const bool plain = WT == kWeightF32 && (mx > FLT_MAX || (mx > 0.f && ex - 13 < -126));
+        bool plain = WT == kWeightF32 && (mx > FLT_MAX || (mx > 0.f && ex - 13 < -126));
+        if constexpr (WT == kWeightF32)
+            plain |= wide_row(min(min(red_low[0], red_low[1]), min(red_low[2], red_low[3])), mx);
         a.xexp[z * a.batch + b] = e + (plain ? kXPlain : 0);
     }
 }
@@ -1808,7 +1832,7 @@ struct TileW<kWeightF32> : TileWBase {
     } next[2][kTileNT];
     int row_off[kTileNT];
     h8 lo[kTileNT][2];
-    uint32_t plain = 0;  // bit j: row j has a chunk the fp16 pairs cannot stand for (see below)
+    uint32_t plain = 0;  // bit j: row j has a chunk the fp16 pairs cannot stand for (any lane group's; see below)
 
     __device__ __forceinline__ void init(const MatmulArgs& a, int o0, int lane_, uint32_t* lds_) {
         base_init(a, o0, (int64_t)a.in_dim * 4, lane_, lds_);
@@ -1826,20 +1850,25 @@ struct TileW<kWeightF32> : TileWBase {
     // The row's largest |w| of the chunk goes to [2^12, 2^13).  d is 2^(e - 13), the
     // other 2^13 joining the batch row's exponent at the end, so that the running
     // sum stays about |w| times the scaled x.  Chunks that reach 2^100 (or hold an infinity), or
-    // whose largest is below 2^-100, leave fp16's or that sum's range: their row is summed in plain fp32.
+    // whose largest is below 2^-100, leave fp16's or that sum's range, and a chunk of a wide range
+    // (kWideLog2) leaves the pairs': their row is summed in plain fp32.
     template <int CC>
     __device__ __forceinline__ void expand(int slot) {
 #pragma unroll
         for (int j = 0; j < kTileNT; ++j) {
             const f4 (&r)[4] = next[slot][j].v;
             float mx = 0.f;
+            uint32_t low = ~0u;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                mx = fmaxf(mx, fmaxf(fmaxf(fabsf(r[i][0]), fabsf(r[i][1])), fmaxf(fabsf(r[i][2]), fabsf(r[i][3]))));
+            for (int i = 0; i < 4; ++i) {
+                const float m4 = fmaxf(fmaxf(fabsf(r[i][0]), fabsf(r[i][1])), fmaxf(fabsf(r[i][2]), fabsf(r[i][3])));
+                mx = fmaxf(mx, m4);
+                low = min(low, __float_as_uint(m4) - 1);
+            }
             mx = lane_group_max(mx);
             const int field = (int)(__float_as_uint(mx) >> 23);
             const int e = min(87, max(-113, field - 139));  // field 126 + ex, mx = f * 2^ex with f in [0.5, 1)
-            if (mx > 0.f && (field - 139 > 87 || field - 139 < -113)) plain |= 1u << j;
+            if (wide_row(low, mx) || (mx > 0.f && (field - 139 > 87 || field - 139 < -113))) plain |= 1u << j;
             const float down = __uint_as_float((uint32_t)(127 - e) << 23);
             d[j] = __uint_as_float((uint32_t)(127 + e - 13) << 23);
 #pragma unroll
@@ -2030,6 +2059,56 @@ __device__ __forceinline__ void tile_products(const MatmulArgs& a, TileW<WT>& w,
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load outlives the loop
 }
 
+// F32 outputs that the fp16 pairs cannot stand for (x rows marked kXPlain, weight
+// rows in `wp`): the wave sums its tile over k0 .. k1 on the fp32 matrix cores, one
+// M tile with such a row at a time, and those outputs replace what it stored.
+// Operand order as in the fp32 form: lane (n, g) brings k = 16 i + 4 g + s to step s.
+__device__ __forceinline__ void plain_products(const MatmulArgs& a, uint32_t wp, int b0, int mt, int o0, int n, int g, int z,
+                                               int k0, int k1, float* dst) {
+    const float* wr[kTileNT];
+#pragma unroll
+    for (int j = 0; j < kTileNT; ++j)
+        wr[j] = static_cast<const float*>(a.w) + (int64_t)min(o0 + 16 * j + n, a.out_dim - 1) * a.in_dim + 4 * g;
+    for (int t = 0; t < mt; ++t) {
+        uint32_t xp = 0;  // bit r: batch row 4 g + r of the tile
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int b = b0 + 16 * t + 4 * g + r;
+            if (b < a.batch && a.xexp[z * a.batch + b] > kXPlain / 2) xp |= 1u << r;
+        }
+        if (!__any(xp | wp)) continue;
+        const float* xr = a.x + (int64_t)min(b0 + 16 * t + n, a.batch - 1) * a.in_dim + 4 * g;
+        f4 acc[kTileNT];
+#pragma unroll
+        for (int j = 0; j < kTileNT; ++j) acc[j] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int k = k0; k < k1; k += 64) {  // ranges are whole chunks
+            f4 xv[4], wv[4][kTileNT];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                xv[i] = *reinterpret_cast<const f4*>(xr + k + 16 * i);
+#pragma unroll
+                for (int j = 0; j < kTileNT; ++j) wv[i][j] = *reinterpret_cast<const f4*>(wr[j] + k + 16 * i);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+#pragma unroll
+                    for (int j = 0; j < kTileNT; ++j)
+                        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[i][s], wv[i][j][s], acc[j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int j = 0; j < kTileNT; ++j) {
+                const int b = b0 + 16 * t + 4 * g + r;
+                const int o = o0 + 16 * j + n;
+                if (b < a.batch && o < a.out_dim && (((xp >> r) | (wp >> j)) & 1))
+                    dst[(int64_t)b * a.out_dim + o] = acc[j][r];
+            }
+    }
+}
+
 template <int WT>
 __global__ __launch_bounds__(kMmThreads, 2) void matmul_tile_kernel(MatmulArgs a) {
     constexpr int NT = kTileNT;
@@ -2092,21 +2171,11 @@ __global__ __launch_bounds__(kMmThreads, 2) void matmul_tile_kernel(MatmulArgs a
             }
         }
     if constexpr (WT == kWeightF32) {
-        // Outputs of rows the fp16 pairs cannot stand for: the same lane's plain sum replaces what it stored.
-        if (plain_any || w.plain) {
-            for (int i = 0; i < 16 * NT; ++i) {
-                const int b = b0 + 16 * (i & 3) + 4 * g + ((i >> 2) & 3);
-                const int j = i >> 4;
-                const int o = o0 + 16 * j + n;
-                if (b >= a.batch || o >= a.out_dim) continue;
-                if (a.xexp[z * a.batch + b] <= kXPlain / 2 && !((w.plain >> j) & 1)) continue;
-                const float* wr = static_cast<const float*>(a.w) + (int64_t)o * a.in_dim;
-                const float* xr = a.x + (int64_t)b * a.in_dim;
-                float s = 0.f;
-                for (int k = 64 * c_begin; k < 64 * c_end; ++k) s = fmaf(wr[k], xr[k], s);
-                dst[(int64_t)b * a.out_dim + o] = s;
-            }
-        }
+        uint32_t wp = w.plain;
+        wp |= __shfl_xor((int)wp, 16);
+        wp |= __shfl_xor((int)wp, 32);
+        plain_any |= wp != 0;
+        if (__any(plain_any)) plain_products(a, wp, b0, mt, o0, n, g, z, 64 * c_begin, 64 * c_end, dst);
     }
 }
 

@@ -397,3 +397,28 @@ def test_tile_form_q4_k_min_term_keeps_the_fp32_sums(torch_mod, gsp, ctx):
     assert np.all(np.abs(x.reshape(batch, -1, 32).sum(-1, dtype=np.float64)).max(-1) > 2.0 ** 23)
     got = _run(torch_mod, gsp, ctx, orc.WTYPE_Q4_K, data, x, in_dim, out_dim)
     assert np.array_equal(got, np.repeat(-x.sum(-1, dtype=np.float64)[:, None], out_dim, 1))
+
+
+@pytest.mark.parametrize("loud", [2.0 ** 18, 1e12], ids=["2p18", "1e12"])
+@pytest.mark.parametrize("shape", [(2112, 4099, 200), (4096, 4100, 260)], ids=["split", "unsplit_tail"])
+def test_tile_form_f32_rows_of_a_wide_range(torch_mod, gsp, ctx, shape, loud):
+    """F32 rows with a few channels 2^18 or 1e12 times the rest, where the other operand is zero: in x, and
+    among the weights of a 64-wide chunk.  fp32 keeps the other channels' bits, a pair scaled to the loud
+    ones would not; the fp32 summation bar holds, and rows without such channels do not change."""
+    in_dim, out_dim, batch = shape
+    print(f"case matmul wide rows {shape} {loud}", flush=True)
+    rng = np.random.default_rng(in_dim + batch)
+    w = (rng.standard_normal((out_dim, in_dim)) / 64).astype(np.float32)
+    x = rng.standard_normal((batch, in_dim)).astype(np.float32)
+    w[:, 100:104] = 0
+    x[:, 1500:1503] = 0
+    plain = _run(torch_mod, gsp, ctx, orc.WTYPE_F32, w, x, in_dim, out_dim)
+    xr, wr = np.array([0, 17, batch - 1]), np.array([3, 1000, out_dim - 1])
+    x[xr, 100:104] *= np.float32(loud)
+    w[wr, 1500:1503] *= np.float32(loud)
+    got = _run(torch_mod, gsp, ctx, orc.WTYPE_F32, w, x, in_dim, out_dim)
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    assert np.all(np.abs(got - x64 @ w64.T) <= 1e-5 * (np.abs(x64) @ np.abs(w64).T) + 1e-7)
+    bx, bw = np.ones(batch, bool), np.ones(out_dim, bool)
+    bx[xr], bw[wr] = False, False
+    assert np.array_equal(got[bx][:, bw], plain[bx][:, bw])
