@@ -58,10 +58,6 @@ constexpr int64_t kSplitNs = 4000;
 constexpr int64_t kMergeRoundNs = 2500;
 constexpr int64_t kMergeRoundPieces = 8;
 
-struct SplitCosts {
-    int64_t tile, unit, split, round;
-};
-
 // Modelled time of the step's decode work cut into pieces of at most `target`
 // tiles: the makespan of LPT-packing the units into `bins` bins, and the longest merge.
 int64_t simulate_split(const std::vector<int32_t>& pages, int32_t heads_kv, int32_t target, int64_t bins,
@@ -333,6 +329,16 @@ int StepPlanner::plan(const PlanPool& pool, const gsp_step_desc* desc, const Pla
                              : pair_cus                    ? (int64_t)kDecodeBinsPerCu * std::max(1, opt.num_cus)
                                                            : (int64_t)std::max(1, opt.num_cus / 4);
     const int64_t sim_bins = pair_cus ? bins_max / kDecodeBinsPerCu : bins_max;
+    // Beside prefill tiles the decode units are not what the step waits for,
+    // and their bins' flat costs in tiles stay.
+    SplitCosts costs{1, kUnitCostPages, kSplitCostPages, 0};
+    if (!any_tiles) {
+        const int64_t elem = pd.kv_dtype == GSP_KV_F32 ? 4 : 2;
+        costs.tile = std::max(kTileFloorNs, tt * (pd.head_dim + pd.v_head_dim) * elem / kCuBytesPerNs);
+        costs.unit = kUnitNs;
+        costs.split = kSplitNs;
+        costs.round = kMergeRoundNs * ((8 * (int64_t)pd.v_head_dim + kDecodeThreads - 1) / kDecodeThreads);
+    }
     int64_t target = 1;
     if (T > 0) {
         if (opt.split_pages_override > 0) {
@@ -340,7 +346,7 @@ int StepPlanner::plan(const PlanPool& pool, const gsp_step_desc* desc, const Pla
         } else if (max_pages <= kWholePairMaxPages && T <= kUnderloadPagesPerBin * bins_max) {
             target = std::max<int64_t>(1, max_pages);  // whole pairs
         } else if (cached_target_ > 0 && cached_heads_kv_ == H && cached_queries_ == total_q &&
-                   cached_bins_ == bins_max && T * 100 >= cached_tasks_ * 97 &&
+                   cached_bins_ == bins_max && cached_costs_ == costs && T * 100 >= cached_tasks_ * 97 &&
                    T * 100 <= cached_tasks_ * 103) {
             target = std::max<int64_t>(cached_target_, min_target);  // engine steps drift slowly
         } else {
@@ -352,16 +358,6 @@ int StepPlanner::plan(const PlanPool& pool, const gsp_step_desc* desc, const Pla
                     const int64_t tot = std::min<int64_t>(desc->token_counts[b], (int64_t)desc->positions[b] + i + 1);
                     if (tot > 0) query_pages_.push_back((int32_t)((tot + tt - 1) / tt));
                 }
-            }
-            // Beside prefill tiles the decode units are not what the step waits for,
-            // and their bins' flat costs in tiles stay.
-            SplitCosts costs{1, kUnitCostPages, kSplitCostPages, 0};
-            if (!any_tiles) {
-                const int64_t elem = pd.kv_dtype == GSP_KV_F32 ? 4 : 2;
-                costs.tile = std::max(kTileFloorNs, tt * (pd.head_dim + pd.v_head_dim) * elem / kCuBytesPerNs);
-                costs.unit = kUnitNs;
-                costs.split = kSplitNs;
-                costs.round = kMergeRoundNs * ((8 * (int64_t)pd.v_head_dim + kDecodeThreads - 1) / kDecodeThreads);
             }
             int64_t best_cost = INT64_MAX;
             for (int32_t cand : kSplitCandidates) {
@@ -379,6 +375,7 @@ int StepPlanner::plan(const PlanPool& pool, const gsp_step_desc* desc, const Pla
             cached_heads_kv_ = H;
             cached_queries_ = total_q;
             cached_bins_ = bins_max;
+            cached_costs_ = costs;
         }
     }
     units_.clear();

@@ -75,6 +75,16 @@ struct StepPlan {
     int32_t tile_pages = 1;
 };
 
+// What a split size is scored by: the cost of a tile, of a unit, of a split
+// piece beyond its tiles and of a merge round.  It depends on the pool's widths
+// and page type.
+struct SplitCosts {
+    int64_t tile = 0, unit = 0, split = 0, round = 0;
+    bool operator==(const SplitCosts& o) const {
+        return tile == o.tile && unit == o.unit && split == o.split && round == o.round;
+    }
+};
+
 class StepPlanner {
 public:
     // Validates `desc` for `pool` (the reference's throws,
@@ -87,12 +97,14 @@ public:
 private:
     int32_t assign_bins(int64_t bins_max, bool pair);
 
-    // Split size chosen for the last step shape (reused while the work drifts < 3%).
+    // Split size chosen for the last step shape (reused while the work drifts < 3%
+    // and nothing else that it was scored by changes).
     int32_t cached_target_ = 0;
     int64_t cached_tasks_ = 0;
     int32_t cached_heads_kv_ = 0;
     int64_t cached_queries_ = 0;
     int64_t cached_bins_ = 0;
+    SplitCosts cached_costs_;
 
     // Scratch reused across steps.
     std::vector<DecodeUnit> units_;    // in the order they were built

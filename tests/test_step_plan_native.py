@@ -78,3 +78,46 @@ def test_step_packer_under_sanitizers(plan_builds, tmp_path, variant):
     assert "ok" in res.stdout.splitlines()[-1], report
     for marker in ("ERROR: AddressSanitizer", "runtime error:", "FAIL "):
         assert marker not in report, report
+
+
+@pytest.fixture(scope="module")
+def sizes_build():
+    subprocess.run(["make", "-C", str(NATIVE), "_build/step_plan_sizes"], check=True, capture_output=True, text=True)
+    return NATIVE / "_build" / "step_plan_sizes"
+
+
+def _sizes(build, path, steps):
+    """{"fresh": [(target, units, slots) per step], "shared": [... of both passes]}"""
+    _write(path, steps)
+    res = subprocess.run([str(build), str(path)], capture_output=True, text=True, timeout=300)
+    assert res.returncode == 0, res.stdout + res.stderr
+    got = {"fresh": [], "shared": []}
+    for ln in res.stdout.splitlines():
+        kind, _, rc, *sizes = ln.split()
+        assert rc == "0", ln
+        got[kind].append(tuple(int(v) for v in sizes))
+    return got
+
+
+def _rows(lens, heads, kv, d, dtype="f32", block_size=16, v_head_dim=None):
+    """A decode step of rows with these token counts."""
+    lens = np.asarray(lens, np.int32)
+    pages = -(-lens // block_size)
+    offsets = np.concatenate([[0], np.cumsum(pages)]).astype(np.int32)
+    step = workloads.small_step(seed=1, rows=len(lens), n_heads=heads, n_kv=kv, head_dim=d, kv_dtype=dtype, ctx_lo=1,
+                                ctx_hi=2, total_blocks=int(pages.sum()) + 1, max_seq_len=65536, block_size=block_size,
+                                v_head_dim=v_head_dim)
+    step.positions, step.token_counts, step.bt_offsets = lens - 1, lens, offsets
+    step.bt_ids = np.arange(pages.sum(), dtype=np.int32)
+    return step
+
+
+def test_split_size_does_not_depend_on_the_pool_packed_before(sizes_build, tmp_path):
+    """One context serves pools that differ only in page type or width: the size chosen for one step is
+    the size a fresh packer chooses, whatever was packed before."""
+    lens = [1500] * 40
+    steps = [_rows(lens, 32, 4, d, dtype, v_head_dim=dv)
+             for d, dtype, dv in [(64, "f16", None), (128, "f32", None), (128, "f16", None), (128, "f32", 64)]]
+    got = _sizes(sizes_build, tmp_path / "steps.bin", steps)
+    assert len(set(got["fresh"])) > 1, got  # the steps' work is the same, their sizes are not
+    assert got["shared"] == got["fresh"] * 2
