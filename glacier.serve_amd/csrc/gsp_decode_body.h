@@ -506,12 +506,13 @@ __device__ __forceinline__ void page_pv(WaveState<D>& st, const PageRegs<D, _Flo
 // rounding error grows with the square root of the longest chain of additions,
 // and long units are the fast ones (16 rows of 16k to 32k tokens, 64/8 heads,
 // fp16: 358 us a layer in 64-page units, 278 in 512-page ones, whose error
-// against float64 was 4.5e-7 in one level against 2.9e-7, and is 2.8e-7 in two).
-// The registers are all in use, so LDS is the second level.  Whole pairs, which
-// the split size never lengthens, and the general shapes, which the longer loop
-// slows by up to 4%, stay in one level, as do mixed steps (2% there, and their
-// units stay short); a flush every 24 fp16 pages takes 0.5%
-// of a step of 256 rows.  fp32 pages add four times per page, fp16 pages once.
+// against float64 was 4.5e-7 in one level against 2.9e-7, and is 2.9e-7 in two;
+// 28 rows of 7000 tokens in whole pairs 4.4e-7 against 2.8e-7).  The registers
+// are all in use, so LDS is the second level.  It takes at most 0.5% of a step
+// (256 rows of up to 8192 fp16 tokens 278.7 and 278.4 us without and with it).
+// The general shapes, which the longer loop slows by up to 4%, stay in one
+// level, as do mixed steps (2% there, and their units stay short).  fp32 pages
+// add four times per page, fp16 pages once.
 template <typename KT>
 constexpr int kFlushPages = sizeof(KT) == 4 ? 8 : 24;  // pages of one wave
 
@@ -639,7 +640,7 @@ __device__ __forceinline__ void load_first_page(PageRegs<D, KT>& pr, const Decod
 // page loop, again with nothing else in flight, and the last split of a pair
 // merges it in that unit's epilogue.  A workgroup's last one or two pieces settle after its
 // final unit.
-// TWO_LEVEL: split units flush their sums (flush_o).
+// TWO_LEVEL: long units flush their sums (flush_o), a path laid out of line.
 template <int D, typename KT, int MODE, bool TWO_LEVEL = MODE == kExact>
 __device__ __forceinline__ void decode_bins_body(const DecodeArgs& a, EpilogueLds<D, kMaxGroupMfma>& sh, int bx,
                                                  int by) {
@@ -716,9 +717,8 @@ __device__ __forceinline__ void decode_bins_body(const DecodeArgs& a, EpilogueLd
         bool flushed = false;  // the wave's LDS part holds pages already
         float m_at = 0.f;      // their max
         if constexpr (TWO_LEVEL) {
-            const bool split = (u.split_info >> 16) > 1;
             while (p < u.page_end) {
-                const int flush_at = split ? min(p + kFlushPages<KT> * kDecodeWaves, u.page_end) : u.page_end;
+                const int flush_at = min(p + kFlushPages<KT> * kDecodeWaves, u.page_end);
                 do {
                     const int pn = p + kDecodeWaves;
                     if (pn < u.page_end && !rb_ready) {
@@ -739,7 +739,7 @@ __device__ __forceinline__ void decode_bins_body(const DecodeArgs& a, EpilogueLd
                     compute_page<D, KT, MODE>(st, rb, q, min(geo.tt, u.ctx - pn * geo.tt), g);
                     p = pnn;
                 } while (p < flush_at);
-                if (p < u.page_end) {
+                if (__builtin_expect(p < u.page_end, 0)) {
                     flush_o<D>(st, sh.o[wave], !flushed, m_at, G, n, g);
                     flushed = true;
                 }
@@ -795,7 +795,7 @@ __device__ __forceinline__ void decode_bins_body(const DecodeArgs& a, EpilogueLd
             sh.m[wave][n] = st.m;
             sh.l[wave][n] = st.l;
         }
-        if (TWO_LEVEL && flushed) {
+        if (TWO_LEVEL && __builtin_expect(flushed, 0)) {
             flush_o<D>(st, sh.o[wave], false, m_at, G, n, g);
         } else {
 #pragma unroll

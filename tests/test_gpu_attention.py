@@ -300,3 +300,34 @@ def test_long_split_units_match_oracle(torch_mod, gsp, ctx, geom, split_pages):
     pool.destroy()
     assert not np.isnan(got).any()
     assert max_err(got, ref) <= 3e-5
+
+
+@pytest.mark.parametrize("dt", ["f16", "f32"])
+def test_long_whole_pairs_sum_in_two_levels(torch_mod, gsp, ctx, dt):
+    """A pair that is not split and has over 100 pages a wave: its error against float64 (2-norms) is that of
+    two-level sums.  One level adds each wave's pages in one chain; measured 4.4e-7 (fp16 pages, 110 pages a
+    wave) and 4.8e-7 (fp32 pages, 31 a wave already) against 2.8e-7 and 3.3e-7 in two."""
+    step = workloads.small_step(seed=70, rows=3, n_heads=32, n_kv=8, head_dim=128, kv_dtype=dt, ctx_lo=6900,
+                                ctx_hi=7100, total_blocks=1400, max_seq_len=8192)
+    print(f"case whole pairs {dt}", flush=True)
+    q, k, v = workloads.host_values(step)
+    pool, keep = to_device_pool(torch_mod, gsp, ctx, step, k, v)
+    ctx.set_decode_path(PATHS["mfma"])
+    try:
+        got = gpu_step(torch_mod, gsp, ctx, step, q, pool, split_pages=512)
+        assert ctx.step_info().split_pairs == 0
+    finally:
+        ctx.set_decode_path(0)
+        pool.destroy()
+    err = mag = 0.0
+    for b in range(step.num_rows):
+        n = int(step.token_counts[b])
+        ids = step.bt_ids[step.bt_offsets[b]: step.bt_offsets[b + 1]]
+        kk = k[ids, 0].astype(np.float64).transpose(1, 0, 2, 3).reshape(8, -1, 128)[:, :n]
+        vv = v[ids, 0].astype(np.float64).transpose(1, 0, 2, 3).reshape(8, -1, 128)[:, :n]
+        sc = np.einsum("hgd,htd->hgt", q[b].astype(np.float64).reshape(8, 4, 128), kk) * step.scale
+        p = np.exp(sc - sc.max(-1, keepdims=True))
+        ref = np.einsum("hgt,htd->hgd", p / p.sum(-1, keepdims=True), vv).reshape(32, 128)
+        err += np.sum((got[b] - ref) ** 2)
+        mag += np.sum(ref ** 2)
+    assert np.sqrt(err / mag) <= 3.8e-7
