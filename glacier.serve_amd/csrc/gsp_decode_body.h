@@ -527,6 +527,7 @@ __device__ __forceinline__ void flush_o(WaveState<D>& st, Rows& o, bool first, f
         for (int r = 0; r < 4; ++r) ar[r] = __shfl(f, 4 * g + r);
     }
     m_at = st.m;
+    static_assert(alignof(EpilogueLds<D, kMaxGroupMfma>) >= sizeof(f4) && D % 4 == 0, "f4 pieces of o");
     int at = 4 * g * D + 4 * n;  // formed here (the empty asm), not kept in a register through the page loop
     asm volatile("" : "+v"(at));
 #pragma unroll

@@ -45,10 +45,11 @@ struct Tile {
     int32_t* counters;
 };
 
-// LDS of the epilogue: the four waves' states (rows of D >= dv floats).
+// LDS of the epilogue: the four waves' states (rows of D >= dv floats, read and
+// written in 16-byte pieces too).
 template <int D, int GMAX>
 struct EpilogueLds {
-    float o[kDecodeWaves][GMAX][D];
+    alignas(16) float o[kDecodeWaves][GMAX][D];
     float m[kDecodeWaves][GMAX];
     float l[kDecodeWaves][GMAX];
     int last;      // the pair counted last is complete: merge it
