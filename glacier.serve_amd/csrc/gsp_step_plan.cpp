@@ -7,6 +7,7 @@
 #include <climits>
 #include <cstring>
 #include <functional>
+#include <iterator>
 
 #include "gsp_status.h"
 
@@ -38,63 +39,168 @@ constexpr int64_t kUnderloadPagesPerBin = 4;
 
 int64_t unit_cost(int64_t pages, bool split) { return pages + kUnitCostPages + (split ? kSplitCostPages : 0); }
 
-// What the split size is scored by, in ns.  A tile of the page stream takes its
-// bytes at a CU's share of the bandwidth (25 bytes/ns), or the latency floor of
-// a tile whose bytes take less.  A split piece costs about 4 us beyond its
-// pages.  The longest merge sits on the step's tail: the merging workgroup loads 8
-// pieces per round for each 256 of the group's outputs, about 2.5 us a round
-// under load (groups of 8 assumed; the group is the caller's at attention time).
-// Fitted to sweeps of 8 to 1024 pages per piece over 13 steps (1 to 64 rows,
-// both page types, head_dim 32 to 128); the sizes it picks measured, against
-// those picked with a flat 3 pages per piece (us a layer): 16 rows of 16k to
-// 32k tokens, 64/8 heads, fp16: 512 pages 278, 64 pages 358; 28/4 heads fp32
-// 64 rows up to 4096: 48 pages 64.4, 32 pages 68.8; one 8192-token row: 32 pages
-// 27.9, 8 pages 33.5; 14/2 heads, 4 rows up to 8192: 24 pages 18.1, 8 pages
-// 20.3.  At worst 42.7 against 41.4 (20 rows, one KV head of width 32).
-constexpr int64_t kCuBytesPerNs = 25;
-constexpr int64_t kTileFloorNs = 400;
-constexpr int64_t kUnitNs = 600;
-constexpr int64_t kSplitNs = 4000;
-constexpr int64_t kMergeRoundNs = 2500;
+// Two scores choose the split size.
+//
+// The flat one: the makespan in pages of LPT-packing the units into the CUs, with
+// unit_cost.  It is all that steps with prefill tiles use (the decode units are not
+// what those wait for), and the general shapes.
+//
+// The modelled time, of decode steps of the compile-time shapes: a size takes the
+// place of the flat choice where it is modelled kMinGainPercent faster, or
+// kMinGainStreamPercent where streaming is at least kStreamPercent of the time (the
+// model's sure part), or where the flat score holds both equal within
+// kFlatTiePercent.  The model:
+//  - a workgroup alone takes `tile` ns a tile (its loads' latency and the CU's
+//    share of the matrix work), kUnitNs a unit and kPieceNs a split piece;
+//  - while all CUs stream, a tile takes a CU `share` ns (the HBM bandwidth divided
+//    by the CUs) and a split piece's publish kPieceShareNs; once CUs run dry the
+//    others stream faster, down to kAloneSharePercent of that;
+//  - the longest merge sits on the step's tail, kMergeRoundNs for each 8 pieces and
+//    256 of the group's outputs (groups of kMergeGroup assumed: the group is the
+//    caller's at attention time);
+//  - kLaunchNs for everything else.
+// Fitted to the times of every candidate on 460 decode steps (1 to 256 rows of up
+// to 32768 tokens, equal and ragged, half of them below 3000; 14/2, 28/4, 32/8 and
+// 64/8 heads; both page types; pages cold), each step's units on the bins that
+// assign_bins gives them.  Over those the chosen size is at worst 1.03 of the flat
+// choice's time.  Against the flat choice (us a layer): 16 rows of 16k to 32k
+// tokens, 64/8 heads fp16, 512 pages 279 (64: 352); 56 rows of 4000, 28/4 fp16,
+// whole pairs 75 (32: 102); 24 rows of 771, 64/8 fp16, whole 18.4 (16: 25.3); 64
+// rows up to 4096, 28/4 fp32, 48 pages 65.8 (32: 69.4).  The flat choice stands for
+// 16 rows of 200 to 575, 32/8 fp16 (16 pages 11.6, whole 12.9) and 256 rows up to
+// 4096, 28/4 fp32 (192 pages 153; whole pairs of up to 256, whose CUs with a single
+// unit leave assign_bins no pairs, 187).
+constexpr int64_t kUnitNs = 1200;
+constexpr int64_t kPieceNs = 1150;
+constexpr int64_t kPieceShareNs = 2850;
+constexpr int64_t kMergeRoundNs = 800;
 constexpr int64_t kMergeRoundPieces = 8;
+constexpr int64_t kMergeGroup = 6;
+constexpr int64_t kLaunchNs = 5800;
+constexpr int64_t kAloneSharePercent = 75;
+constexpr int64_t kMinGainPercent = 15;
+constexpr int64_t kMinGainStreamPercent = 4;
+constexpr int64_t kStreamPercent = 80;
+constexpr int64_t kFlatTiePercent = 2;
 
-// Modelled time of the step's decode work cut into pieces of at most `target`
-// tiles: the makespan of LPT-packing the units into `bins` bins, and the longest merge.
-int64_t simulate_split(const std::vector<int32_t>& pages, int32_t heads_kv, int32_t target, int64_t bins,
-                       const SplitCosts& cost_of, std::vector<int64_t>& count, std::vector<int64_t>& heap) {
-    int32_t pieces = 1;
-    // count[2s] whole pairs of s pages, count[2s + 1] split pieces of s pages.
+// The units that pieces of at most `target` tiles give, as counts by size:
+// count[2s] whole pairs of s tiles, count[2s + 1] split pieces of s tiles.
+struct UnitSizes {
+    int32_t longest = 0;  // tiles
+    int32_t pieces = 1;   // of the pair cut into most
+    int64_t units = 0;
+};
+
+UnitSizes count_units(const std::vector<int32_t>& pages, int32_t heads_kv, int32_t target, std::vector<int64_t>& count) {
+    UnitSizes n;
     count.assign(2 * ((size_t)target + 1), 0);
-    int32_t longest = 0;
     for (int32_t P : pages) {
         const int32_t ns = std::min((P + target - 1) / target, gsp::kMaxSplits);
         const int32_t base = P / ns, extra = P % ns;
         const int sp = ns > 1 ? 1 : 0;
-        pieces = std::max(pieces, ns);
+        n.pieces = std::max(n.pieces, ns);
         // Pieces of base + 1 pages exist only when extra > 0, and then base < target.
         if (extra) count[2 * ((size_t)base + 1) + sp] += (int64_t)extra * heads_kv;
         count[2 * (size_t)base + sp] += (int64_t)(ns - extra) * heads_kv;
-        longest = std::max(longest, base + (extra ? 1 : 0));
+        n.longest = std::max(n.longest, base + (extra ? 1 : 0));
+        n.units += (int64_t)ns * heads_kv;
     }
-    heap.clear();
-    for (int32_t s = longest; s >= 1; --s) {
-        for (int sp = 1; sp >= 0; --sp) {
-            const int64_t cost = s * cost_of.tile + cost_of.unit + (sp == 1 ? cost_of.split : 0);
-            for (int64_t c = count[2 * (size_t)s + sp]; c > 0; --c) {
-                if ((int64_t)heap.size() < bins) {
-                    heap.push_back(-cost);  // min-heap through negated loads
-                    std::push_heap(heap.begin(), heap.end());
-                } else {
-                    std::pop_heap(heap.begin(), heap.end());
-                    heap.back() -= cost;
-                    std::push_heap(heap.begin(), heap.end());
-                }
+    return n;
+}
+
+// Calls fn(s, split, number) for every size, longest first, split pieces first.
+template <typename F>
+void each_size(const UnitSizes& n, const std::vector<int64_t>& count, F&& fn) {
+    for (int32_t s = n.longest; s >= 1; --s)
+        for (int sp = 1; sp >= 0; --sp)
+            if (count[2 * (size_t)s + sp]) fn(s, sp == 1, count[2 * (size_t)s + sp]);
+}
+
+// LPT of the units into `bins` bins (assign_bins' order and costs); returns the makespan in pages.
+int64_t pack_units(const UnitSizes& n, const std::vector<int64_t>& count, int64_t bins, std::vector<PlanBin>& bin,
+                   std::vector<uint64_t>& heap) {
+    bins = std::min(bins, n.units);
+    bin.assign((size_t)bins, PlanBin{});
+    // Min-heap of load << 32 | bin; the least loaded bin takes the next unit in place.
+    heap.resize((size_t)bins);
+    for (size_t b = 0; b < heap.size(); ++b) heap[b] = b;
+    const size_t size = heap.size();
+    uint64_t worst = 0;
+    each_size(n, count, [&](int32_t s, bool split, int64_t c) {
+        const uint64_t cost = (uint64_t)unit_cost(s, split) << 32;
+        for (; c > 0; --c) {
+            const uint64_t key = heap[0] + cost;
+            bin[key & 0xFFFFFFFFu].add(s, split);
+            worst = std::max(worst, key);
+            size_t at = 0;
+            for (size_t child = 1; child < size; child = 2 * at + 1) {
+                child += child + 1 < size && heap[child + 1] < heap[child];
+                if (key <= heap[child]) break;
+                heap[at] = heap[child];
+                at = child;
             }
+            heap[at] = key;
+        }
+    });
+    return (int64_t)(worst >> 32);
+}
+
+// Modelled time of a decode step whose units are in `cu` as pack_units left them
+// over the `cus` CUs, on the bins that assign_bins gives them.
+int64_t merge_ns(const UnitSizes& n, const SplitCosts& k) {
+    return n.pieces > 1 ? k.round * ((n.pieces + kMergeRoundPieces - 1) / kMergeRoundPieces) : 0;
+}
+
+// No modelled time of the step is below this.
+int64_t least_ns(const UnitSizes& n, const SplitCosts& k, int64_t pages, int64_t cus) {
+    return kLaunchNs + pages * k.share / cus + merge_ns(n, k);
+}
+
+struct StepTime {
+    int64_t ns = INT64_MAX;
+    int64_t stream = 0;  // the part of it that the HBM streams
+};
+
+StepTime step_time(const UnitSizes& n, const std::vector<int64_t>& count, const SplitCosts& k, int64_t cus,
+                   std::vector<PlanBin>& cu,
+                   std::vector<PlanBin>& wg, std::vector<uint64_t>& heap, std::vector<int64_t>& share) {
+    const auto alone = [&](const PlanBin& b) { return b.pages * k.tile + b.units * kUnitNs + b.splits * kPieceNs; };
+    int64_t longest = 0;  // the last workgroup, were every tile to come at its own pace
+    bool paired = n.units >= 2 * cus;
+    for (const PlanBin& b : cu) paired = paired && b.units >= 2;
+    if (paired) {
+        // assign_bins deals a CU's units to its two workgroups, about half each.
+        for (const PlanBin& b : cu)
+            longest = std::max(longest, std::max(alone(b) / 2, b.longest * k.tile + kUnitNs + (b.splits ? kPieceNs : 0)));
+    } else {
+        // A workgroup per unit, or LPT over the workgroups; c and c + cus share a CU.
+        if (n.units <= 2 * cus) {
+            wg.clear();
+            each_size(n, count, [&](int32_t s, bool split, int64_t c) {
+                PlanBin b;
+                b.add(s, split);
+                wg.insert(wg.end(), (size_t)c, b);
+            });
+        } else {
+            pack_units(n, count, 2 * cus, wg, heap);
+        }
+        cu.assign((size_t)cus, PlanBin{});
+        for (size_t b = 0; b < wg.size(); ++b) {
+            longest = std::max(longest, alone(wg[b]));
+            PlanBin& c = cu[b % (size_t)cus];
+            c.pages += wg[b].pages;
+            c.splits += wg[b].splits;
         }
     }
-    int64_t worst = 0;
-    for (int64_t x : heap) worst = std::max(worst, -x);
-    return pieces > 1 ? worst + cost_of.round * ((pieces + kMergeRoundPieces - 1) / kMergeRoundPieces) : worst;
+    share.clear();
+    for (const PlanBin& b : cu) share.push_back(b.pages * k.share + b.splits * kPieceShareNs);
+    std::sort(share.begin(), share.end());
+    int64_t stream = 0, done = 0;
+    for (int64_t i = 0; i < cus; ++i) {
+        stream += (share[(size_t)i] - done) * std::max(100 * (cus - i) / cus, kAloneSharePercent);
+        done = share[(size_t)i];
+    }
+    return {kLaunchNs + std::max(stream / 100, longest) + merge_ns(n, k), stream / 100};
 }
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
@@ -329,15 +435,15 @@ int StepPlanner::plan(const PlanPool& pool, const gsp_step_desc* desc, const Pla
                              : pair_cus                    ? (int64_t)kDecodeBinsPerCu * std::max(1, opt.num_cus)
                                                            : (int64_t)std::max(1, opt.num_cus / 4);
     const int64_t sim_bins = pair_cus ? bins_max / kDecodeBinsPerCu : bins_max;
-    // Beside prefill tiles the decode units are not what the step waits for,
-    // and their bins' flat costs in tiles stay.
-    SplitCosts costs{1, kUnitCostPages, kSplitCostPages, 0};
-    if (!any_tiles) {
-        const int64_t elem = pd.kv_dtype == GSP_KV_F32 ? 4 : 2;
-        costs.tile = std::max(kTileFloorNs, tt * (pd.head_dim + pd.v_head_dim) * elem / kCuBytesPerNs);
-        costs.unit = kUnitNs;
-        costs.split = kSplitNs;
-        costs.round = kMergeRoundNs * ((8 * (int64_t)pd.v_head_dim + kDecodeThreads - 1) / kDecodeThreads);
+    // Two workgroups per CU, no prefill tiles, and a shape the decode kernels have
+    // at compile time (what the model was fitted to): the split size is modelled in time.
+    SplitCosts costs;
+    const bool modelled = pair_cus && tileable;
+    if (modelled) {
+        const int64_t bytes = tt * (pd.head_dim + pd.v_head_dim) * (pd.kv_dtype == GSP_KV_F32 ? 4 : 2);
+        costs.tile = 85 + bytes / (pd.kv_dtype == GSP_KV_F32 ? 38 : 60);
+        costs.share = std::max<int64_t>(1, bytes * 2 / 63);
+        costs.round = kMergeRoundNs * ((kMergeGroup * pd.v_head_dim + kDecodeThreads - 1) / kDecodeThreads);
     }
     int64_t target = 1;
     if (T > 0) {
@@ -359,17 +465,39 @@ int StepPlanner::plan(const PlanPool& pool, const gsp_step_desc* desc, const Pla
                     if (tot > 0) query_pages_.push_back((int32_t)((tot + tt - 1) / tt));
                 }
             }
-            int64_t best_cost = INT64_MAX;
-            for (int32_t cand : kSplitCandidates) {
+            constexpr int kNone = -1;
+            int64_t flat[std::size(kSplitCandidates)];
+            StepTime time[std::size(kSplitCandidates)];
+            int first = kNone, last = kNone, best = kNone, fastest = kNone;
+            for (int i = 0; i < (int)std::size(kSplitCandidates); ++i) {
+                const int32_t cand = kSplitCandidates[i];
                 if (cand < min_target) continue;
                 if (T / cand > 16 * bins_max) continue;  // far too many units to be competitive
-                const int64_t c = simulate_split(query_pages_, H, cand, sim_bins, costs, sim_count_, sim_heap_);
-                if (c <= best_cost) {  // ties go to the larger split (fewer units)
-                    best_cost = c;
-                    target = cand;
+                if (first == kNone) first = i;
+                last = i;
+                const UnitSizes n = count_units(query_pages_, H, cand, sim_count_);
+                flat[i] = pack_units(n, sim_count_, sim_bins, sim_cu_, sim_heap_);
+                // Ties go to the larger split (fewer units).
+                if (best == kNone || flat[i] <= flat[best]) best = i;
+                if (modelled && (flat[i] <= flat[best] * (100 + kFlatTiePercent) / 100 ||
+                                 least_ns(n, costs, T, sim_bins) <= time[fastest].ns)) {
+                    time[i] = step_time(n, sim_count_, costs, sim_bins, sim_cu_, sim_wg_, sim_heap_, bin_load_);
+                    if (fastest == kNone || time[i].ns <= time[fastest].ns) fastest = i;
                 }
                 if (cand >= max_pages) break;  // larger candidates give the same units
             }
+            if (modelled && best != kNone) {
+                const StepTime& t = time[fastest];
+                const int64_t gain = t.stream * 100 >= t.ns * kStreamPercent ? kMinGainStreamPercent : kMinGainPercent;
+                if (t.ns * 100 < time[best].ns * (100 - gain)) {
+                    best = fastest;
+                } else {
+                    const int64_t tie = flat[best] * (100 + kFlatTiePercent) / 100;
+                    for (int i = first; i <= last; ++i)
+                        if (flat[i] <= tie && time[i].ns < time[best].ns) best = i;
+                }
+            }
+            if (best != kNone) target = kSplitCandidates[best];
             cached_target_ = (int32_t)target;
             cached_tasks_ = T;
             cached_heads_kv_ = H;

@@ -75,13 +75,22 @@ struct StepPlan {
     int32_t tile_pages = 1;
 };
 
-// What a split size is scored by: the cost of a tile, of a unit, of a split
-// piece beyond its tiles and of a merge round.  It depends on the pool's widths
-// and page type.
+// What a split size is modelled by, in ns (0: it is not modelled): a tile for a
+// workgroup alone, a tile at a CU's share of the bandwidth, a merge round.  They
+// depend on the pool's widths and page type.
 struct SplitCosts {
-    int64_t tile = 0, unit = 0, split = 0, round = 0;
-    bool operator==(const SplitCosts& o) const {
-        return tile == o.tile && unit == o.unit && split == o.split && round == o.round;
+    int64_t tile = 0, share = 0, round = 0;
+    bool operator==(const SplitCosts& o) const { return tile == o.tile && share == o.share && round == o.round; }
+};
+
+// What a workgroup or CU holds in a modelled schedule.
+struct PlanBin {
+    int64_t pages = 0, units = 0, splits = 0, longest = 0;
+    void add(int64_t s, bool split) {
+        pages += s;
+        units += 1;
+        splits += split;
+        longest = longest < s ? s : longest;
     }
 };
 
@@ -121,7 +130,9 @@ private:
     std::vector<int32_t> q_ctx_;
     std::vector<int32_t> query_pages_;
     std::vector<int32_t> voffs_, vids_;  // row tables in kernel pages (pool pages above 16 tokens)
-    std::vector<int64_t> sim_count_, sim_heap_;
+    std::vector<int64_t> sim_count_;
+    std::vector<PlanBin> sim_cu_, sim_wg_;
+    std::vector<uint64_t> sim_heap_;
 };
 
 }  // namespace gsp

@@ -115,9 +115,42 @@ def _rows(lens, heads, kv, d, dtype="f32", block_size=16, v_head_dim=None):
 def test_split_size_does_not_depend_on_the_pool_packed_before(sizes_build, tmp_path):
     """One context serves pools that differ only in page type or width: the size chosen for one step is
     the size a fresh packer chooses, whatever was packed before."""
-    lens = [1500] * 40
+    lens = [7000] * 28
     steps = [_rows(lens, 32, 4, d, dtype, v_head_dim=dv)
              for d, dtype, dv in [(64, "f16", None), (128, "f32", None), (128, "f16", None), (128, "f32", 64)]]
     got = _sizes(sizes_build, tmp_path / "steps.bin", steps)
     assert len(set(got["fresh"])) > 1, got  # the steps' work is the same, their sizes are not
     assert got["shared"] == got["fresh"] * 2
+
+
+# Steps of equal rows and the time of a layer measured for some split sizes (us, MI355X, cold pages).  `bar`:
+# the size that the packer's flat score takes, which the modelled one may replace only where it is no slower.
+MEASURED = [
+    # rows, tokens, heads, KV heads, head_dim, page type, bar, {pages: us}
+    (1, 667, 28, 4, 128, "f16", 8, {8: 10.3, 12: 11.0, 24: 12.9, 48: 14.3}),
+    (3, 393, 28, 4, 128, "f32", 8, {8: 12.5, 16: 15.7, 32: 17.5}),
+    (5, 450, 64, 8, 128, "f32", 8, {8: 14.1, 16: 16.5, 32: 19.5}),
+    (6, 469, 32, 8, 128, "f16", 8, {8: 10.2, 16: 11.4, 32: 11.5}),
+    (18, 456, 28, 4, 128, "f32", 12, {8: 18.6, 12: 15.7, 16: 18.4, 32: 20.2}),
+    (27, 329, 28, 4, 128, "f32", 20, {8: 18.4, 12: 15.9, 20: 15.8, 24: 17.9}),
+    (15, 771, 32, 8, 128, "f16", 48, {16: 15.6, 32: 15.1, 48: 15.1, 64: 16.8}),
+    (21, 934, 32, 8, 128, "f32", 24, {20: 34.5, 24: 34.5, 32: 42.5, 48: 42.3, 64: 39.0}),
+    (29, 12489, 28, 4, 128, "f32", 64, {48: 260.3, 64: 259.6, 128: 271.6, 256: 235.9, 512: 231.4, 1024: 377.3}),
+    (2, 22234, 14, 2, 64, "f16", 24, {16: 25.6, 24: 21.7, 32: 19.8, 48: 25.8, 96: 27.7}),
+    # Measured faster than the flat choice by a fifth and more: the modelled size takes its place.
+    (33, 439, 64, 8, 128, "f16", None, {12: 25.7, 16: 24.2, 24: 24.1, 32: 19.3}),
+    (135, 437, 14, 2, 64, "f16", None, {12: 18.0, 16: 17.6, 24: 17.6, 32: 11.9}),
+    (1, 3502, 64, 8, 128, "f16", None, {8: 21.4, 12: 18.5, 16: 16.3, 32: 16.8, 64: 21.4}),
+    (7, 29216, 64, 8, 128, "f16", None, {48: 177.7, 128: 165.1, 256: 142.5, 512: 138.8, 1024: 233.4}),
+]
+
+
+def test_split_sizes_against_measured_steps(sizes_build, tmp_path):
+    steps = [_rows([n] * rows, heads, kv, d, dt) for rows, n, heads, kv, d, dt, _, _ in MEASURED]
+    got = _sizes(sizes_build, tmp_path / "steps.bin", steps)["fresh"]
+    for case, (size, _, _) in zip(MEASURED, got):
+        times = case[-1]
+        assert size in times, (case, size)
+        bar = case[-2]
+        limit = 1.03 * times[bar] if bar else 1.05 * min(times.values())
+        assert times[size] <= limit, (case, size)
