@@ -484,7 +484,7 @@ __device__ __forceinline__ void page_pv(WaveState<D>& st, const PageRegs<D, _Flo
     // block 4c + i takes B[token 4g + kk][col] = V[4g + kk][64c + 4n + i],
     // i.e. element i of the lane's four V pieces.
     // P arrives times 2^12 (compute_page), so p_lo of a typical probability is a
-    // normal fp16 number: the matrix cores flush fp16 subnormals.
+    // normal fp16 number with all its bits.
     typedef _Float16 h8 __attribute__((ext_vector_type(8)));
     const h4 ph = __builtin_convertvector(p, h4);
     const h4 pl = __builtin_convertvector(p - __builtin_convertvector(ph, f4), h4);

@@ -1506,7 +1506,6 @@ __global__ __launch_bounds__(kMmThreads) void matmul_split_x_tile_kernel(MatmulA
 // few KB of LDS that belong to the wave alone: no barrier, LDS serves a wave's
 // accesses in order.
 typedef uint32_t u2v __attribute__((ext_vector_type(2)));
-typedef uint32_t u3v __attribute__((ext_vector_type(3)));
 
 __device__ __forceinline__ h2 splat2(_Float16 v) { return h2{v, v}; }
 

@@ -23,9 +23,9 @@
 //   - Q: per query token (the lane's S column), at load;
 //   - fp32 K, V pages: per key row, while the page is staged into LDS;
 //     fp16 pages are exact in fp16 and enter as they are (x_lo = 0);
-//   - P: times 2^12, so that p_lo stays a normal fp16 number (the matrix
-//     cores flush fp16 subnormals; an unscaled p_lo of a typical probability
-//     would be one, and P would keep only 11 bits).  P = 2^(s - m) is taken
+//   - P: times 2^12, so that p_lo stays a normal fp16 number (an unscaled p_lo
+//     of a typical probability would be subnormal and hold fewer than its 11
+//     bits).  P = 2^(s - m) is taken
 //     against a max m that lags the running max by at most 2^3 (the O
 //     rescale is skipped until a row grows further), so P' < 2^15.
 // S = K_hi.Q_hi + K_hi.Q_lo + K_lo.Q_hi (the K_lo.Q_lo term is ~2^-22
