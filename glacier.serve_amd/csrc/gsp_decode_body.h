@@ -510,9 +510,10 @@ __device__ __forceinline__ void page_pv(WaveState<D>& st, const PageRegs<D, _Flo
 // 28 rows of 7000 tokens in whole pairs 4.4e-7 against 2.8e-7).  The registers
 // are all in use, so LDS is the second level.  It takes at most 0.5% of a step
 // (256 rows of up to 8192 fp16 tokens 278.7 and 278.4 us without and with it).
-// The general shapes, which the longer loop slows by up to 4%, stay in one
-// level, as do mixed steps (2% there, and their units stay short).  fp32 pages
-// add four times per page, fp16 pages once.
+// Steps without units that long take the kernel without it (launch_exact).  The
+// general shapes, which the longer loop slows by up to 4%, stay in one level, as
+// do mixed steps (2% there, and their units stay short).  fp32 pages add four
+// times per page, fp16 pages once.
 template <typename KT>
 constexpr int kFlushPages = sizeof(KT) == 4 ? 8 : 24;  // pages of one wave
 
@@ -641,8 +642,8 @@ __device__ __forceinline__ void load_first_page(PageRegs<D, KT>& pr, const Decod
 // page loop, again with nothing else in flight, and the last split of a pair
 // merges it in that unit's epilogue.  A workgroup's last one or two pieces settle after its
 // final unit.
-// TWO_LEVEL: long units flush their sums (flush_o), a path laid out of line.
-template <int D, typename KT, int MODE, bool TWO_LEVEL = MODE == kExact>
+// TWO_LEVEL: units of more than kFlushPages pages a wave flush their sums (flush_o), a path laid out of line.
+template <int D, typename KT, int MODE, bool TWO_LEVEL>
 __device__ __forceinline__ void decode_bins_body(const DecodeArgs& a, EpilogueLds<D, kMaxGroupMfma>& sh, int bx,
                                                  int by) {
 

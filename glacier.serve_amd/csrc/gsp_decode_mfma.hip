@@ -5,15 +5,27 @@
 namespace gsp {
 namespace {
 
-template <int D, typename KT, int MODE>
+template <int D, typename KT, int MODE, bool TWO_LEVEL>
 __global__ __launch_bounds__(kDecodeThreads, D >= 256 ? 1 : 2) void paged_decode_mfma_kernel(DecodeArgs a) {
     __shared__ EpilogueLds<D, kMaxGroupMfma> sh;
-    decode_bins_body<D, KT, MODE>(a, sh, blockIdx.x, blockIdx.y);
+    decode_bins_body<D, KT, MODE, TWO_LEVEL>(a, sh, blockIdx.x, blockIdx.y);
 }
 
-template <int D, typename KT, int MODE>
+template <int D, typename KT, int MODE, bool TWO_LEVEL = false>
 void launch_one(dim3 grid, const DecodeArgs& a, hipStream_t stream) {
-    hipLaunchKernelGGL((paged_decode_mfma_kernel<D, KT, MODE>), grid, dim3(kDecodeThreads), 0, stream, a);
+    hipLaunchKernelGGL((paged_decode_mfma_kernel<D, KT, MODE, TWO_LEVEL>), grid, dim3(kDecodeThreads), 0, stream, a);
+}
+
+// Units that never flush take the kernel without the second level: the results are
+// the same bit for bit, and a unit's start and end are shorter there (136 rows of 11
+// to 259 tokens, 64/8 heads fp32: 33.2 us a layer against 34.0; 4 rows of 20 to 300,
+// 28/4 fp32: 11.95 against 12.27).
+template <int D, typename KT>
+void launch_exact(dim3 grid, const DecodeArgs& a, hipStream_t stream) {
+    if (a.unit_tiles > kFlushPages<KT> * kDecodeWaves)
+        launch_one<D, KT, kExact, true>(grid, a, stream);
+    else
+        launch_one<D, KT, kExact>(grid, a, stream);
 }
 
 template <typename KT>
@@ -25,9 +37,9 @@ hipError_t launch_typed(dim3 grid, const DecodeArgs& a, hipStream_t stream) {
         return hipErrorInvalidValue;
     if (d == dv && a.block_size == kBlockSize && (d == 64 || d == 128)) {
         if (d == 128)
-            launch_one<128, KT, kExact>(grid, a, stream);
+            launch_exact<128, KT>(grid, a, stream);
         else
-            launch_one<64, KT, kExact>(grid, a, stream);
+            launch_exact<64, KT>(grid, a, stream);
     } else if (d < 1 || dv < 1 || d > 256 || dv > 256 || a.block_size < 1 || a.block_size > kTileTokens) {
         return hipErrorInvalidValue;
     } else if (d % 2 || dv % 2) {

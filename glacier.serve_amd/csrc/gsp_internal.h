@@ -46,6 +46,7 @@ struct DecodeArgs {
     int32_t total_q;
     int32_t num_slots;     // partial slots per tile
     int32_t slot_heads;    // heads per partial slot: min(group, 16)
+    int32_t unit_tiles;    // no unit of the step has more tiles
 };
 
 struct PrefillArgs {

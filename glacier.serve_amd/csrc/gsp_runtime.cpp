@@ -1518,6 +1518,7 @@ int attention_launch(gsp_ctx* ctx, const gsp_pool* pool, int32_t layer, int32_t 
     a.total_q = ctx->info.total_q;
     a.num_slots = slots;
     a.slot_heads = slot_heads;
+    a.unit_tiles = ctx->info.pages_per_split;
     const int f16 = d.kv_dtype == GSP_KV_F16;
     gsp::PrefillArgs p;
     p.k_pool = a.k_pool;

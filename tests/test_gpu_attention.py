@@ -331,3 +331,32 @@ def test_long_whole_pairs_sum_in_two_levels(torch_mod, gsp, ctx, dt):
         err += np.sum((got[b] - ref) ** 2)
         mag += np.sum(ref ** 2)
     assert np.sqrt(err / mag) <= 3.8e-7
+
+
+@pytest.mark.parametrize("dt,pages", [("f32", 32), ("f16", 96)])
+@pytest.mark.parametrize("d,heads,nkv", [(128, 28, 4), (64, 14, 2)])
+def test_one_and_two_level_kernels_agree(torch_mod, gsp, ctx, dt, pages, d, heads, nkv):
+    """A step whose longest unit is what the one-level kernel takes (8 fp32 or 24 fp16 pages a wave) and the same
+    row beside one that is a page longer, which takes the two-level kernel: the row's output is equal bit for bit,
+    and both rows match the oracle."""
+    step = workloads.small_step(seed=pages + d, rows=2, n_heads=heads, n_kv=nkv, head_dim=d, kv_dtype=dt,
+                                ctx_lo=16 * pages, ctx_hi=16 * pages, total_blocks=256, max_seq_len=4096)
+    step.token_counts = np.array([16 * pages, 16 * pages + 1], np.int32)
+    step.positions = step.token_counts - 1
+    step.bt_offsets = np.array([0, pages, 2 * pages + 1], np.int32)
+    step.bt_ids = np.random.default_rng(pages).permutation(256)[: 2 * pages + 1].astype(np.int32)
+    print(f"case one and two levels {dt} d{d}", flush=True)
+    q, k, v = workloads.host_values(step)
+    pool, keep = to_device_pool(torch_mod, gsp, ctx, step, k, v)
+    ctx.set_decode_path(PATHS["mfma"])
+    try:
+        both = gpu_step(torch_mod, gsp, ctx, step, q, pool, split_pages=512)
+        one = workloads.Step(step.name, heads, nkv, d, dt, 256, 4096, step.positions[:1], step.token_counts[:1],
+                             step.bt_offsets[:2], step.bt_ids[:pages], None, step.seed)
+        alone = gpu_step(torch_mod, gsp, ctx, one, q[:1], pool, split_pages=pages)
+        assert ctx.step_info().pages_per_split == pages
+    finally:
+        ctx.set_decode_path(0)
+        pool.destroy()
+    assert np.array_equal(alone[0], both[0])
+    assert max_err(both, oracle_step(step, q, k, v, threads=threads())) <= 3e-5
