@@ -180,7 +180,7 @@ KQ_SHAPES = [
     (2048, 2048, 100),
     (512, 4100, 65),
     (3584, 3584, 256),
-    (18944, 1024, 200),  # rows longer than the pre-pass keeps in registers (Qwen2.5-7B's down projection)
+    (18944, 1024, 200),  # Qwen2.5-7B's down projection width: K ranges in the tile form (Q4_K), one in the fp16 form
 ]
 
 
@@ -422,3 +422,22 @@ def test_tile_form_f32_rows_of_a_wide_range(torch_mod, gsp, ctx, shape, loud):
     bx, bw = np.ones(batch, bool), np.ones(out_dim, bool)
     bx[xr], bw[wr] = False, False
     assert np.array_equal(got[bx][:, bw], plain[bx][:, bw])
+
+
+# One K range of more than 8192 values, which the tile form's pre-pass reads twice instead of keeping it.
+@pytest.mark.parametrize("w_type,in_dim", [(orc.WTYPE_F32, 8256), (orc.WTYPE_Q8_0, 8256), (orc.WTYPE_Q4_K, 8448),
+                                           (orc.WTYPE_Q6_K, 8448)], ids=lambda v: str(v))
+def test_tile_form_pre_pass_of_long_ranges(torch_mod, gsp, ctx, w_type, in_dim):
+    """264 tiles on 256 CUs: K is not split, and the row's largest value lies past the first 8192."""
+    out_dim, batch = 4100, 450
+    rng = np.random.default_rng(in_dim + w_type)
+    if w_type in (orc.WTYPE_Q4_K, orc.WTYPE_Q6_K):
+        data, wm = _kquant_weights(rng, w_type, out_dim, in_dim)
+    else:
+        data, wm = _weights(rng, w_type, out_dim, in_dim)
+    print(f"case long pre-pass type={w_type}", flush=True)
+    x = rng.standard_normal((batch, in_dim)).astype(np.float32)
+    x[:, 8200] *= np.float32(40.0)
+    got = _run(torch_mod, gsp, ctx, w_type, data, x, in_dim, out_dim)
+    x64, wm = x.astype(np.float64), np.asarray(wm, np.float64)
+    assert np.all(np.abs(got - x64 @ wm.T) <= 1e-5 * (np.abs(x64) @ np.abs(wm).T) + 1e-7)
