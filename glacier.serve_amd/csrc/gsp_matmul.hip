@@ -1292,7 +1292,7 @@ __global__ __launch_bounds__(kMmThreads, 2) void matmul_q6k_f16_small_kernel(Mat
 // staged in LDS serves all four waves and two N tiles, and a wave expands its
 // own rows' words to fp16 operands in registers once per chunk of 64 k and uses
 // each for four M tiles.  Measured at 1024 rows of 4096 x 4096 (us): Q8_0 177 ->
-// 107, Q4_K 185 -> 101, Q6_K 194 -> 136, F32 279 -> 173, about 700 TFLOP/s of
+// 107, Q4_K 185 -> 101, Q6_K 194 -> 136, F32 279 -> 168, about 700 TFLOP/s of
 // fp16 matrix steps; what is left is instruction issue (a chunk of Q6_K is
 // 48 matrix steps and 130 vector instructions a wave; dropping the expansion
 // or the scaling takes it to 128 us each, the barriers nothing).
@@ -1323,8 +1323,7 @@ __global__ __launch_bounds__(kMmThreads, 2) void matmul_q6k_f16_small_kernel(Mat
 //     element, or 2^-38 of the scale's largest where that is more, and the lo x
 //     lo product (at most 2^-22, typically 2^-25 of the term) is left out;
 //     operands whose range is too wide for that, or that leave fp16's, go to
-//     plain_products (kWideLog2, kXPlain; the check costs 4 of 62 us at 256
-//     rows).  Against float64 the products are closer than the fp32 form's
+//     plain_products (kWideLog2, kXPlain).  Against float64 the products are closer than the fp32 form's
 //     (4096 x 4096 at 256 rows: 8.4e-7 -> 1.6e-7): a running sum rounds once a
 //     chunk instead of once per four k.
 // K is split over ranges only where the tiles leave CUs idle; the ranges' sums
@@ -1356,10 +1355,11 @@ struct KOrder {
 constexpr int kXPlain = 1 << 16;
 // A scaled pair holds an element to 2^-23 of itself or 2^-38 of the scale's
 // largest, whichever is more (the matrix cores keep fp16 subnormals).  F32
-// operands are wide, and summed in plain fp32, when four neighbours lie below
-// 2^-kWideLog2 of the largest and are not all zero: every group of four then
-// keeps 22 bits of its own largest.  (Among 4096 normal values beside a channel
-// 12 times as loud that happens once in 10^9 rows.)
+// operands are wide, and summed in plain fp32, when a group of neighbours (four of
+// a row of x; of weights the eight of a 64-wide chunk that one lane has from each
+// 32) lies below 2^-kWideLog2 of the largest and is not all zero: otherwise every
+// group keeps 22 bits of its own largest.  (Among 4096 normal values beside a
+// channel 12 times as loud that happens once in 10^9 rows.)
 constexpr int kWideLog2 = 16;
 // `low`: the least, over the groups, of the bits of a group's largest magnitude minus one (zero groups wrap to the top).
 __device__ __forceinline__ bool wide_row(uint32_t low, float mx) {
@@ -1831,7 +1831,7 @@ struct TileW<kWeightF32> : TileWBase {
     } next[2][kTileNT];
     int row_off[kTileNT];
     h8 lo[kTileNT][2];
-    uint32_t plain = 0;  // bit j: row j has a chunk the fp16 pairs cannot stand for (any lane group's; see below)
+    uint32_t range[kTileNT] = {};  // see expand; each lane group of the row has its part
 
     __device__ __forceinline__ void init(const MatmulArgs& a, int o0, int lane_, uint32_t* lds_) {
         base_init(a, o0, (int64_t)a.in_dim * 4, lane_, lds_);
@@ -1849,25 +1849,33 @@ struct TileW<kWeightF32> : TileWBase {
     // The row's largest |w| of the chunk goes to [2^12, 2^13).  d is 2^(e - 13), the
     // other 2^13 joining the batch row's exponent at the end, so that the running
     // sum stays about |w| times the scaled x.  Chunks that reach 2^100 (or hold an infinity), or
-    // whose largest is below 2^-100, leave fp16's or that sum's range, and a chunk of a wide range
-    // (kWideLog2) leaves the pairs': their row is summed in plain fp32.
+    // with weights below 2^-100, leave fp16's or that sum's range, and a chunk of a wide range
+    // (kWideLog2) leaves the pairs': their row is summed in plain fp32.  The check is in whole
+    // numbers on purpose: as compares and a mask it cost 4.5 of 62 us (256 rows of 4096 x 4096),
+    // with groups of four weights 2.5; as it is, nothing.
     template <int CC>
     __device__ __forceinline__ void expand(int slot) {
 #pragma unroll
         for (int j = 0; j < kTileNT; ++j) {
             const f4 (&r)[4] = next[slot][j].v;
             float mx = 0.f;
-            uint32_t low = ~0u;
+            uint32_t low = ~0u;  // see wide_row; the groups are the lane's halves of the chunk
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float m4 = fmaxf(fmaxf(fabsf(r[i][0]), fabsf(r[i][1])), fmaxf(fabsf(r[i][2]), fabsf(r[i][3])));
-                mx = fmaxf(mx, m4);
-                low = min(low, __float_as_uint(m4) - 1);
+            for (int i = 0; i < 2; ++i) {
+                float m8 = 0.f;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) m8 = fmaxf(m8, fabsf(r[2 * i + (q >> 2)][q & 3]));
+                mx = fmaxf(mx, m8);
+                low = min(low, __float_as_uint(m8) - 1);
             }
             mx = lane_group_max(mx);
             const int field = (int)(__float_as_uint(mx) >> 23);
             const int e = min(87, max(-113, field - 139));  // field 126 + ex, mx = f * 2^ex with f in [0.5, 1)
-            if (wide_row(low, mx) || (mx > 0.f && (field - 139 > 87 || field - 139 < -113))) plain |= 1u << j;
+            // The distance, as bits, from the chunk's largest (at least 2^-84) to its least group, or
+            // from 2^84 to its largest: 2^16 apart or more and the pairs cannot stand for the row.
+            const uint32_t m = __float_as_uint(mx);
+            range[j] = max(range[j], max(__builtin_elementwise_sub_sat(max(m, (127u - 84) << 23), low),
+                                         __builtin_elementwise_sub_sat(m, (127u + 84) << 23)));
             const float down = __uint_as_float((uint32_t)(127 - e) << 23);
             d[j] = __uint_as_float((uint32_t)(127 + e - 13) << 23);
 #pragma unroll
@@ -2170,9 +2178,14 @@ __global__ __launch_bounds__(kMmThreads, 2) void matmul_tile_kernel(MatmulArgs a
             }
         }
     if constexpr (WT == kWeightF32) {
-        uint32_t wp = w.plain;
-        wp |= __shfl_xor((int)wp, 16);
-        wp |= __shfl_xor((int)wp, 32);
+        uint32_t wp = 0;  // bit j: weight row 16 j + n
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            uint32_t m = w.range[j];
+            m = max(m, (uint32_t)__shfl_xor((int)m, 16));
+            m = max(m, (uint32_t)__shfl_xor((int)m, 32));
+            wp |= (uint32_t)(m >= ((uint32_t)kWideLog2 << 23)) << j;
+        }
         plain_any |= wp != 0;
         if (__any(plain_any)) plain_products(a, wp, b0, mt, o0, n, g, z, 64 * c_begin, 64 * c_end, dst);
     }

@@ -968,9 +968,9 @@ constexpr int64_t kMatmulSmallMinOutputs = 16384;
 //     gain, at a larger summation error than the small form's, so none take it.
 //   Q6_K above 64 rows: 4096 x 4096 at 1024 194 -> 136, 3584 x 3584 at 300 73
 //     -> 62; 1024 x 4864 at 1000 68.0 -> 68.4, 3584 x 3584 at 128 37 -> 38.5.
-//   F32: 4096 x 4096 at 1024 279 -> 173, at 256 88 -> 62, 3584 x 3584 at 128
-//     46.9 -> 37.3, 18944 x 3584 at 64 109 -> 105, 4096 x 16384 at 64 88 -> 66;
-//     at the line 4096 x 1024 at 300 37.6 -> 37.8; up to 48 rows the fp32 form has
+//   F32: 4096 x 4096 at 1024 278 -> 168, at 256 86 -> 58, 3584 x 3584 at 128
+//     46.5 -> 34.8, 18944 x 3584 at 64 109 -> 70, 4096 x 16384 at 64 89 -> 63;
+//     at the line 4096 x 1024 at 300 37.6 -> 37.6; up to 48 rows the fp32 form has
 //     fewer M tiles to run, this one does not: 8192 x 16384 at 48 147 -> 153, 4096
 //     x 32768 at 32 130 -> 130.
 static bool use_matmul_tile(int32_t w_type, int64_t in_dim, int64_t out_dim, int64_t batch) {
@@ -1017,9 +1017,9 @@ int gsp_matmul_batch(gsp_ctx* ctx, int32_t w_type, const void* w_dev, const floa
         // Splits: K ranges of at least 8 chunks, about one workgroup per CU (4096 x
         // 4096 at 100 rows Q4_K, 64 tiles: 47.6 us unsplit, 27.4 in 4 ranges, 31.1 in
         // 8; F32 at 256 rows, 128 tiles: 60 us in 2, 67 in 3, where half the CUs run
-        // two workgroups, and 3584 x 3584 at 128 rows, 56 tiles: 37.3 us in 4, 47.3 in 5,
+        // two workgroups, and 3584 x 3584 at 128 rows, 56 tiles: 34.6 us in 4, 45.4 in 5,
         // so F32 takes more than one per CU only where it would not split otherwise
-        // (3584 x 18944 at 64 rows, 148 tiles: 101 us unsplit, 97 in 2); 3584 x 18944 at 64 rows Q4_K, 148 tiles: 47.3 and 45.8 in 2;
+        // (4096 x 3584 at 300 rows, 140 tiles: 86.9 us in 2, 92.1 unsplit); 3584 x 18944 at 64 rows Q4_K, 148 tiles: 47.3 and 45.8 in 2;
         // 4096 x 4096 at 512 rows, 256 tiles, 58.0 and 58.4 in 2; at 1024 rows 100 and 112).
         const int64_t chunks = in_dim / 64;
         const int64_t groups = (batch + 63) / 64;
