@@ -46,41 +46,34 @@ int64_t unit_cost(int64_t pages, bool split) { return pages + kUnitCostPages + (
 // what those wait for), and the general shapes.
 //
 // The modelled time, of decode steps of the compile-time shapes: a size takes the
-// place of the flat choice where it is modelled kMinGainPercent faster, or
-// kMinGainStreamPercent where streaming is at least kStreamPercent of the time (the
-// model's sure part), or where the flat score holds both equal within
-// kFlatTiePercent.  The model:
+// place of the flat choice where it is modelled kMinGainPercent faster, or where the
+// flat score holds both equal within kFlatTiePercent.  The model:
 //  - a workgroup alone takes `tile` ns a tile (its loads' latency and the CU's
 //    share of the matrix work), kUnitNs a unit and kPieceNs a split piece;
 //  - while all CUs stream, a tile takes a CU `share` ns (the HBM bandwidth divided
 //    by the CUs) and a split piece's publish kPieceShareNs; once CUs run dry the
 //    others stream faster, down to kAloneSharePercent of that;
-//  - the longest merge sits on the step's tail, kMergeRoundNs for each 8 pieces and
-//    256 of the group's outputs (groups of kMergeGroup assumed: the group is the
-//    caller's at attention time);
-//  - kLaunchNs for everything else.
-// Fitted to the times of every candidate on 460 decode steps (1 to 256 rows of up
+//  - the longest merge sits on the step's tail (merge_ns), and kLaunchNs stand for
+//    everything else.
+// Fitted to the times of every candidate on 390 decode steps (1 to 256 rows of up
 // to 32768 tokens, equal and ragged, half of them below 3000; 14/2, 28/4, 32/8 and
 // 64/8 heads; both page types; pages cold), each step's units on the bins that
-// assign_bins gives them.  Over those the chosen size is at worst 1.03 of the flat
-// choice's time.  Against the flat choice (us a layer): 16 rows of 16k to 32k
-// tokens, 64/8 heads fp16, 512 pages 279 (64: 352); 56 rows of 4000, 28/4 fp16,
-// whole pairs 75 (32: 102); 24 rows of 771, 64/8 fp16, whole 18.4 (16: 25.3); 64
-// rows up to 4096, 28/4 fp32, 48 pages 65.8 (32: 69.4).  The flat choice stands for
-// 16 rows of 200 to 575, 32/8 fp16 (16 pages 11.6, whole 12.9) and 256 rows up to
-// 4096, 28/4 fp32 (192 pages 153; whole pairs of up to 256, whose CUs with a single
-// unit leave assign_bins no pairs, 187).
+// assign_bins gives them.  Over those the chosen size is 3% faster than the flat
+// choice, at worst 1.04 of its time.  Against the flat choice (us a layer): 16 rows
+// of 16k to 32k tokens, 64/8 heads fp16, 512 pages 279 (64: 352); 56 rows of 4000,
+// 28/4 fp16, whole pairs 75 (32: 102); 24 rows of 771, 64/8 fp16, whole 18.4 (16:
+// 25.3); 64 rows up to 4096, 28/4 fp32, 48 pages 65.8 (32: 69.4); 3 rows of 1600,
+// 32/8 fp16, 16 pages 12.9 (12: 14.7).  The flat choice stands for 16 rows of 200 to
+// 575, 32/8 fp16 (16 pages 11.6, whole 12.9) and 256 rows up to 4096, 28/4 fp32 (192
+// pages 153; whole pairs of up to 256, whose CUs with a single unit leave
+// assign_bins no pairs, 187).  On 70 steps of 32-wide heads the model was up to 1.9
+// slower, so the general shapes keep the flat score.
 constexpr int64_t kUnitNs = 1200;
 constexpr int64_t kPieceNs = 1150;
-constexpr int64_t kPieceShareNs = 2850;
-constexpr int64_t kMergeRoundNs = 800;
-constexpr int64_t kMergeRoundPieces = 8;
-constexpr int64_t kMergeGroup = 6;
-constexpr int64_t kLaunchNs = 5800;
+constexpr int64_t kPieceShareNs = 2000;
+constexpr int64_t kLaunchNs = 4800;
 constexpr int64_t kAloneSharePercent = 75;
-constexpr int64_t kMinGainPercent = 15;
-constexpr int64_t kMinGainStreamPercent = 4;
-constexpr int64_t kStreamPercent = 80;
+constexpr int64_t kMinGainPercent = 6;
 constexpr int64_t kFlatTiePercent = 2;
 
 // The units that pieces of at most `target` tiles give, as counts by size:
@@ -147,18 +140,25 @@ int64_t pack_units(const UnitSizes& n, const std::vector<int64_t>& count, int64_
 
 // Modelled time of a decode step whose units are in `cu` as pack_units left them
 // over the `cus` CUs, on the bins that assign_bins gives them.
-int64_t merge_ns(const UnitSizes& n, const SplitCosts& k) {
-    return n.pieces > 1 ? k.round * ((n.pieces + kMergeRoundPieces - 1) / kMergeRoundPieces) : 0;
+// The merge of the pair cut into most pieces, on the step's tail.  The wide form
+// (gsp_epilogue.h) takes up to 256 / group pieces, 8 a round (measured over whole
+// pairs: 2 us at 4, 6 at 10, 10 at 18, 14 at 34), the general one more of them in
+// less time each (9 us at 40, 15 at 90).  The group is the caller's at attention
+// time: between 32 pieces (groups of 8) and 64 (groups of 4) either may run, `most`
+// counts the longer.
+int64_t merge_ns(int32_t pieces, bool most) {
+    if (pieces <= 1) return 0;
+    return pieces <= (most ? 64 : 32) ? 300 + 1600 * ((pieces + 7) / 8) + 230 * pieces : 5300 + 110 * pieces;
 }
 
 // No modelled time of the step is below this.
 int64_t least_ns(const UnitSizes& n, const SplitCosts& k, int64_t pages, int64_t cus) {
-    return kLaunchNs + pages * k.share / cus + merge_ns(n, k);
+    return kLaunchNs + pages * k.share / cus + merge_ns(n.pieces, true);
 }
 
 struct StepTime {
-    int64_t ns = INT64_MAX;
-    int64_t stream = 0;  // the part of it that the HBM streams
+    int64_t ns = INT64_MAX;     // with the longer merge
+    int64_t least = INT64_MAX;  // with the shorter one
 };
 
 StepTime step_time(const UnitSizes& n, const std::vector<int64_t>& count, const SplitCosts& k, int64_t cus,
@@ -200,7 +200,8 @@ StepTime step_time(const UnitSizes& n, const std::vector<int64_t>& count, const 
         stream += (share[(size_t)i] - done) * std::max(100 * (cus - i) / cus, kAloneSharePercent);
         done = share[(size_t)i];
     }
-    return {kLaunchNs + std::max(stream / 100, longest) + merge_ns(n, k), stream / 100};
+    const int64_t ns = kLaunchNs + std::max(stream / 100, longest);
+    return {ns + merge_ns(n.pieces, true), ns + merge_ns(n.pieces, false)};
 }
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
@@ -442,8 +443,7 @@ int StepPlanner::plan(const PlanPool& pool, const gsp_step_desc* desc, const Pla
     if (modelled) {
         const int64_t bytes = tt * (pd.head_dim + pd.v_head_dim) * (pd.kv_dtype == GSP_KV_F32 ? 4 : 2);
         costs.tile = 85 + bytes / (pd.kv_dtype == GSP_KV_F32 ? 38 : 60);
-        costs.share = std::max<int64_t>(1, bytes * 2 / 63);
-        costs.round = kMergeRoundNs * ((kMergeGroup * pd.v_head_dim + kDecodeThreads - 1) / kDecodeThreads);
+        costs.share = std::max<int64_t>(1, bytes / 29);
     }
     int64_t target = 1;
     if (T > 0) {
@@ -487,14 +487,12 @@ int StepPlanner::plan(const PlanPool& pool, const gsp_step_desc* desc, const Pla
                 if (cand >= max_pages) break;  // larger candidates give the same units
             }
             if (modelled && best != kNone) {
-                const StepTime& t = time[fastest];
-                const int64_t gain = t.stream * 100 >= t.ns * kStreamPercent ? kMinGainStreamPercent : kMinGainPercent;
-                if (t.ns * 100 < time[best].ns * (100 - gain)) {
+                if (time[fastest].ns * 100 < time[best].least * (100 - kMinGainPercent)) {
                     best = fastest;
                 } else {
                     const int64_t tie = flat[best] * (100 + kFlatTiePercent) / 100;
                     for (int i = first; i <= last; ++i)
-                        if (flat[i] <= tie && time[i].ns < time[best].ns) best = i;
+                        if (flat[i] <= tie && time[i].ns < time[best].least) best = i;
                 }
             }
             if (best != kNone) target = kSplitCandidates[best];

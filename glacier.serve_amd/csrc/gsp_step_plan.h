@@ -76,11 +76,11 @@ struct StepPlan {
 };
 
 // What a split size is modelled by, in ns (0: it is not modelled): a tile for a
-// workgroup alone, a tile at a CU's share of the bandwidth, a merge round.  They
-// depend on the pool's widths and page type.
+// workgroup alone, and at a CU's share of the bandwidth.  They depend on the pool's
+// widths and page type.
 struct SplitCosts {
-    int64_t tile = 0, share = 0, round = 0;
-    bool operator==(const SplitCosts& o) const { return tile == o.tile && share == o.share && round == o.round; }
+    int64_t tile = 0, share = 0;
+    bool operator==(const SplitCosts& o) const { return tile == o.tile && share == o.share; }
 };
 
 // What a workgroup or CU holds in a modelled schedule.
