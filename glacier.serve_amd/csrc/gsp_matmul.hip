@@ -1293,9 +1293,10 @@ __global__ __launch_bounds__(kMmThreads, 2) void matmul_q6k_f16_small_kernel(Mat
 // own rows' words to fp16 operands in registers once per chunk of 64 k and uses
 // each for four M tiles.  Measured at 1024 rows of 4096 x 4096 (us): Q8_0 177 ->
 // 107, Q4_K 185 -> 101, Q6_K 194 -> 136, F32 279 -> 168, about 700 TFLOP/s of
-// fp16 matrix steps; what is left is instruction issue (a chunk of Q6_K is
-// 48 matrix steps and 130 vector instructions a wave; dropping the expansion
-// or the scaling takes it to 128 us each, the barriers nothing).
+// fp16 matrix steps.  Matrix cores busy 22 to 36%, vector issue 35 to 41%, waves
+// waiting on memory or barriers 26 to 28%, but 45% for Q6_K, whose loop over four M
+// tiles reloads spilled registers (a chunk of Q6_K is 48 matrix steps and 130 vector
+// instructions a wave).
 //
 // x comes from matmul_split_x_tile_kernel as scaled fp16 pairs in the order the
 // operands are read, so a chunk of the workgroup's 64 rows is 16 KB in one

@@ -1019,8 +1019,9 @@ int gsp_matmul_batch(gsp_ctx* ctx, int32_t w_type, const void* w_dev, const floa
         // 8; F32 at 256 rows, 128 tiles: 60 us in 2, 67 in 3, where half the CUs run
         // two workgroups, and 3584 x 3584 at 128 rows, 56 tiles: 34.6 us in 4, 45.4 in 5,
         // so F32 takes more than one per CU only where it would not split otherwise
-        // (4096 x 3584 at 300 rows, 140 tiles: 86.9 us in 2, 92.1 unsplit); 3584 x 18944 at 64 rows Q4_K, 148 tiles: 47.3 and 45.8 in 2;
-        // 4096 x 4096 at 512 rows, 256 tiles, 58.0 and 58.4 in 2; at 1024 rows 100 and 112).
+        // (4096 x 3584 at 300 rows, 140 tiles: 86.9 us in 2, 92.1 unsplit); 3584 x 18944
+        // at 64 rows Q4_K, 148 tiles: 47.3 and 45.8 in 2; 4096 x 4096 at 512 rows, 256
+        // tiles, 58.0 and 58.4 in 2; at 1024 rows 100 and 112).
         const int64_t chunks = in_dim / 64;
         const int64_t groups = (batch + 63) / 64;
         const int64_t tiles = groups * ((out_dim + gsp::matmul_tile_rows() - 1) / gsp::matmul_tile_rows());

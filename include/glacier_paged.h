@@ -253,12 +253,12 @@ int gsp_rope_write_step_ex(gsp_ctx* ctx, gsp_pool* pool, int32_t layer, int32_t 
  * fp16 quant and fp32 scale) and sums are fp32.  Q8_0, Q4_K and Q6_K
  * products with at least 16384 outputs (batch x out_dim) at up to 64 batch
  * rows, or at least 196608 outputs, and F32 products of at least 1.5e9
- * multiply-adds above 64 rows (4e9 at 49 to 64), take x as a scaled fp16 pair on
- * the fp16 matrix cores (other products keep x in fp32): each element then
- * carries ~22 significant bits, and elements below 2^-15 of their row's largest
- * |x| an absolute error of at most 2^-37 of it; every finite x stays finite.
- * Those F32 products scale their weights the same way by each 64 weights of a
- * row.  There, x rows and weight rows whose range is too wide for that (four
+ * multiply-adds and 1024 output columns above 64 rows (of 4e9 multiply-adds at 49
+ * to 64), take x as a scaled fp16 pair on the fp16 matrix cores (other products
+ * keep x in fp32): each element then carries ~22 significant bits, and elements
+ * below 2^-15 of their row's largest |x| an absolute error of at most 2^-37 of it;
+ * every finite x stays finite.  Those F32 products scale their weights the same
+ * way by each 64 weights of a row.  There, x rows and weight rows whose range is too wide for that (four
  * neighbours of x, or eight of 64 weights, that are not all zero and lie below
  * 2^-16 of the largest), and rows with infinities or magnitudes outside 2^-100
  * .. 2^100, have their outputs summed in plain fp32.
