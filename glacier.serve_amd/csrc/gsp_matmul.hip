@@ -2067,53 +2067,98 @@ __device__ __forceinline__ void tile_products(const MatmulArgs& a, TileW<WT>& w,
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load outlives the loop
 }
 
-// F32 outputs that the fp16 pairs cannot stand for (x rows marked kXPlain, weight
-// rows in `wp`): the wave sums its tile over k0 .. k1 on the fp32 matrix cores, one
-// M tile with such a row at a time, and those outputs replace what it stored.
-// Operand order as in the fp32 form: lane (n, g) brings k = 16 i + 4 g + s to step s.
-__device__ __forceinline__ void plain_products(const MatmulArgs& a, uint32_t wp, int b0, int mt, int o0, int n, int g, int z,
-                                               int k0, int k1, float* dst) {
-    const float* wr[kTileNT];
+// MB x NB blocks of 16 x 16 outputs (M tiles from batch row b, N tiles from weight
+// row o) over k0 .. k1 on the fp32 matrix cores.  Operand order as
+// in the fp32 form: lane (n, g) brings k = 16 i + 4 g + s to step s; the next 64 k
+// load while these are multiplied.
+template <int MB, int NB>
+__device__ __forceinline__ void plain_block(const MatmulArgs& a, int b, int o, int n, int g, int k0, int k1, f4 (&acc)[MB][NB]) {
+    const float *xr[MB], *wr[NB];
 #pragma unroll
-    for (int j = 0; j < kTileNT; ++j)
-        wr[j] = static_cast<const float*>(a.w) + (int64_t)min(o0 + 16 * j + n, a.out_dim - 1) * a.in_dim + 4 * g;
-    for (int t = 0; t < mt; ++t) {
-        uint32_t xp = 0;  // bit r: batch row 4 g + r of the tile
+    for (int p = 0; p < MB; ++p) xr[p] = a.x + (int64_t)min(b + 16 * p + n, a.batch - 1) * a.in_dim + 4 * g;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int b = b0 + 16 * t + 4 * g + r;
-            if (b < a.batch && a.xexp[z * a.batch + b] > kXPlain / 2) xp |= 1u << r;
+    for (int j = 0; j < NB; ++j)
+        wr[j] = static_cast<const float*>(a.w) + (int64_t)min(o + 16 * j + n, a.out_dim - 1) * a.in_dim + 4 * g;
+    f4 xv[2][MB][4], wv[2][NB][4];
+    auto load = [&](int slot, int k) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int p = 0; p < MB; ++p) xv[slot][p][i] = *reinterpret_cast<const f4*>(xr[p] + k + 16 * i);
+#pragma unroll
+            for (int j = 0; j < NB; ++j) wv[slot][j][i] = *reinterpret_cast<const f4*>(wr[j] + k + 16 * i);
         }
-        if (!__any(xp | wp)) continue;
-        const float* xr = a.x + (int64_t)min(b0 + 16 * t + n, a.batch - 1) * a.in_dim + 4 * g;
-        f4 acc[kTileNT];
+    };
 #pragma unroll
-        for (int j = 0; j < kTileNT; ++j) acc[j] = f4{0.f, 0.f, 0.f, 0.f};
-        for (int k = k0; k < k1; k += 64) {  // ranges are whole chunks
-            f4 xv[4], wv[4][kTileNT];
+    for (int p = 0; p < MB; ++p)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                xv[i] = *reinterpret_cast<const f4*>(xr + k + 16 * i);
+        for (int j = 0; j < NB; ++j) acc[p][j] = f4{0.f, 0.f, 0.f, 0.f};
+    auto products = [&](int slot) {
 #pragma unroll
-                for (int j = 0; j < kTileNT; ++j) wv[i][j] = *reinterpret_cast<const f4*>(wr[j] + k + 16 * i);
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int p = 0; p < MB; ++p)
+#pragma unroll
+                    for (int j = 0; j < NB; ++j)
+                        acc[p][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[slot][p][i][s], wv[slot][j][i][s], acc[p][j], 0, 0, 0);
+    };
+    load(0, k0);
+    for (int k = k0; k < k1; k += 128) {  // ranges are whole chunks
+        if (k + 64 < k1) load(1, k + 64);
+        products(0);
+        if (k + 64 >= k1) break;
+        if (k + 128 < k1) load(0, k + 128);
+        products(1);
+    }
+}
+
+// F32 outputs that the fp16 pairs cannot stand for: bit m of `xm` marks batch row b0
+// + m, bit i of wm[w] weight row o0 + 32 w + i.  The workgroup sums the blocks with
+// such a row in plain fp32, 2 x 2 blocks to each wave in turn, and those outputs
+// replace what was stored.  256 rows of 4096 x 4096: one such weight row 84 us (58
+// without), one such row of x 102, all of them 174 (the fp32 form 87): the loads'
+// address work bounds it, 16 rows a load.
+__device__ __forceinline__ void plain_products(const MatmulArgs& a, uint64_t xm, const uint32_t (&wm)[4], int b0, int mt,
+                                               int o0, int lane, int wave, int k0, int k1, float* dst) {
+    const int n = lane & 15, g = lane >> 4;
+    int turn = 0;
+    for (int at = 0; at < 8; ++at) {
+        const int t = 2 * (at >> 2), pair = at & 3;  // M tiles t, t + 1 and N tiles 2 pair, 2 pair + 1
+        if (t >= mt) break;
+        const uint32_t xb = (uint32_t)(xm >> (16 * t)), wb = wm[pair];  // 32 rows each
+        if (!(xb | wb) || (turn++ & 3) != wave) continue;
+        const int b = b0 + 16 * t, o = o0 + 32 * pair;
+        auto store = [&](int p, int j, const f4& sum) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int m = 16 * p + 4 * g + r, i = 16 * j + n;
+                if (b + m < a.batch && o + i < a.out_dim && (((xb >> m) | (wb >> i)) & 1))
+                    dst[(int64_t)(b + m) * a.out_dim + o + i] = sum[r];
             }
+        };
+        // Rows of one M (N) tile only: half the block.
+        if (!wb && (!(xb >> 16) || !(xb & 0xFFFFu))) {
+            const int p = xb >> 16 ? 1 : 0;
+            f4 acc[1][2];
+            plain_block(a, b + 16 * p, o, n, g, k0, k1, acc);
+            store(p, 0, acc[0][0]);
+            store(p, 1, acc[0][1]);
+        } else if (!xb && (!(wb >> 16) || !(wb & 0xFFFFu))) {
+            const int j = wb >> 16 ? 1 : 0;
+            f4 acc[2][1];
+            plain_block(a, b, o + 16 * j, n, g, k0, k1, acc);
+            store(0, j, acc[0][0]);
+            store(1, j, acc[1][0]);
+        } else {
+            f4 acc[2][2];
+            plain_block(a, b, o, n, g, k0, k1, acc);
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int p = 0; p < 2; ++p)
 #pragma unroll
-                for (int s = 0; s < 4; ++s)
-#pragma unroll
-                    for (int j = 0; j < kTileNT; ++j)
-                        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[i][s], wv[i][j][s], acc[j], 0, 0, 0);
+                for (int j = 0; j < 2; ++j) store(p, j, acc[p][j]);
         }
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int j = 0; j < kTileNT; ++j) {
-                const int b = b0 + 16 * t + 4 * g + r;
-                const int o = o0 + 16 * j + n;
-                if (b < a.batch && o < a.out_dim && (((xp >> r) | (wp >> j)) & 1))
-                    dst[(int64_t)b * a.out_dim + o] = acc[j][r];
-            }
     }
 }
 
@@ -2163,7 +2208,6 @@ __global__ __launch_bounds__(kMmThreads, 2) void matmul_tile_kernel(MatmulArgs a
     // Lane holds batch rows b0 + 16 t + 4 g + r of weight rows o0 + 16 j + n.
     float* dst = a.split_out ? a.split_out + (int64_t)z * a.batch * a.out_dim : a.y;
     constexpr int kExtra = WT == kWeightF32 ? 13 : 0;
-    bool plain_any = false;
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -2171,7 +2215,6 @@ __global__ __launch_bounds__(kMmThreads, 2) void matmul_tile_kernel(MatmulArgs a
             const int b = b0 + 16 * t + 4 * g + r;
             if (b >= a.batch) continue;
             const int e = a.xexp[z * a.batch + b];
-            if (WT == kWeightF32 && e > kXPlain / 2) plain_any = true;
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
                 const int o = o0 + 16 * j + n;
@@ -2179,16 +2222,24 @@ __global__ __launch_bounds__(kMmThreads, 2) void matmul_tile_kernel(MatmulArgs a
             }
         }
     if constexpr (WT == kWeightF32) {
-        uint32_t wp = 0;  // bit j: weight row 16 j + n
+        // Rows the fp16 pairs cannot stand for, as masks: the batch group's 64 and each wave's 32.
+        uint32_t rows = 0;
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
             uint32_t m = w.range[j];
             m = max(m, (uint32_t)__shfl_xor((int)m, 16));
             m = max(m, (uint32_t)__shfl_xor((int)m, 32));
-            wp |= (uint32_t)(m >= ((uint32_t)kWideLog2 << 23)) << j;
+            rows |= ((uint32_t)__ballot(m >= ((uint32_t)kWideLog2 << 23)) & 0xFFFFu) << (16 * j);
         }
-        plain_any |= wp != 0;
-        if (__any(plain_any)) plain_products(a, wp, b0, mt, o0, n, g, z, 64 * c_begin, 64 * c_end, dst);
+        const uint64_t xm = __ballot(b0 + lane < a.batch && a.xexp[z * a.batch + b0 + lane] > kXPlain / 2);
+        // Words of their own: other waves' last direct loads of x may still be landing.  The barrier also
+        // orders a wave's stores above before another's below.
+        __shared__ uint32_t wide_rows[4];
+        if (lane == 0) wide_rows[wave] = rows;
+        __syncthreads();
+        const uint32_t wm[4] = {wide_rows[0], wide_rows[1], wide_rows[2], wide_rows[3]};
+        if (xm || wm[0] | wm[1] | wm[2] | wm[3])
+            plain_products(a, xm, wm, b0, mt, bx * 64 * NT, lane, wave, 64 * c_begin, 64 * c_end, dst);
     }
 }
 

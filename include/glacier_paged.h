@@ -258,10 +258,10 @@ int gsp_rope_write_step_ex(gsp_ctx* ctx, gsp_pool* pool, int32_t layer, int32_t 
  * keep x in fp32): each element then carries ~22 significant bits, and elements
  * below 2^-15 of their row's largest |x| an absolute error of at most 2^-37 of it;
  * every finite x stays finite.  Those F32 products scale their weights the same
- * way by each 64 weights of a row.  There, x rows and weight rows whose range is too wide for that (four
- * neighbours of x, or eight of 64 weights, that are not all zero and lie below
- * 2^-16 of the largest), and rows with infinities or magnitudes outside 2^-100
- * .. 2^100, have their outputs summed in plain fp32.
+ * way by each 64 weights of a row.  There, rows of x and of weights whose range is
+ * too wide for that (four neighbours of x, or eight of 64 weights, that are not
+ * all zero and lie below 2^-16 of the largest), and rows with infinities or
+ * magnitudes outside 2^-100 .. 2^100, have their outputs summed in plain fp32.
  * Results are the same bit for bit on every call, captured or not.
  * Graph capture: run the product, or a larger one of its kind, once before
  * capturing it (a capture that finds the workspace too small fails with

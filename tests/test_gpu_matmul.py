@@ -413,7 +413,8 @@ def test_tile_form_f32_rows_of_a_wide_range(torch_mod, gsp, ctx, shape, loud):
     w[:, 100:104] = 0
     x[:, 1500:1503] = 0
     plain = _run(torch_mod, gsp, ctx, orc.WTYPE_F32, w, x, in_dim, out_dim)
-    xr, wr = np.array([0, 17, batch - 1]), np.array([3, 1000, out_dim - 1])
+    # Both and one M tile of a pair, either one; N tiles likewise.
+    xr, wr = np.array([0, 17, 80, batch - 1]), np.array([3, 1000, 2000, 3000, 3016, out_dim - 1])
     x[xr, 100:104] *= np.float32(loud)
     w[wr, 1500:1503] *= np.float32(loud)
     got = _run(torch_mod, gsp, ctx, orc.WTYPE_F32, w, x, in_dim, out_dim)
