@@ -1459,22 +1459,27 @@ __global__ __launch_bounds__(kMmThreads) void matmul_split_x_tile_kernel(MatmulA
             *reinterpret_cast<h8*>(dst + (g * 16 + m) * 8 + 512) = lo;
         }
         if constexpr (WT == kWeightQ4_K) {
-            // Four consecutive threads hold a sub-block's 32 values.  Its fp32 sum is three
-            // halves (11 + 11 + 2 bits, so all of it) in the lane group's slot 4 * (sub-block % 2)
-            // of the row's sums operand, [64-row group][super-block][M tile][lane][8 halves].
+            // Four consecutive threads hold a sub-block's 32 values, eight the two of a lane group
+            // (ranges are whole super-blocks).  A sum's fp32 value is three halves (11 + 11 + 2
+            // bits); the lane group's operand is both sums' first halves, then their second and
+            // third ones and zeros, [64-row group][super-block][M tile][lane][8 halves].
             sm += __shfl_xor(sm, 1);
             sm += __shfl_xor(sm, 2);
-            if ((i & 3) == 0) {
-                const float v = sm * (1.0f / (1 << kXBlockSumLog2));
-                const bool inf = __builtin_isinf(v);  // rides on its first half alone
-                const _Float16 v0 = (_Float16)v;
-                const float r1 = inf ? 0.f : (v - (float)v0) * (1.0f / kSumScale1);
-                const _Float16 v1 = (_Float16)r1;
-                const _Float16 v2 = (_Float16)((r1 - (float)v1) * (kSumScale1 / kSumScale2));
-                const int sub = (k >> 5) & 7;
-                _Float16* sd = reinterpret_cast<_Float16*>(a.xsum) +
-                               (((row0 >> 2) + (k >> 8)) * 4 + tile) * 512 + ((sub >> 1) * 16 + m) * 8;
-                *reinterpret_cast<h4v*>(sd + 4 * (sub & 1)) = h4v{v0, v1, v2, (_Float16)0.f};
+            const float other = __shfl_xor(sm, 4);
+            if ((i & 7) == 0) {
+                h8 ops = {};
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const float v = (q ? other : sm) * (1.0f / (1 << kXBlockSumLog2));
+                    const bool inf = __builtin_isinf(v);  // rides on its first half alone
+                    ops[q] = (_Float16)v;
+                    const float r1 = inf ? 0.f : (v - (float)ops[q]) * (1.0f / kSumScale1);
+                    ops[2 + q] = (_Float16)r1;
+                    ops[4 + q] = (_Float16)((r1 - (float)ops[2 + q]) * (kSumScale1 / kSumScale2));
+                }
+                _Float16* sd = reinterpret_cast<_Float16*>(a.xsum) + (((row0 >> 2) + (k >> 8)) * 4 + tile) * 512 +
+                               (((k >> 6) & 3) * 16 + m) * 8;
+                *reinterpret_cast<h8*>(sd) = ops;
             }
         }
     };
@@ -1514,7 +1519,7 @@ __device__ __forceinline__ h2 splat2(_Float16 v) { return h2{v, v}; }
 __device__ __forceinline__ h8 sums_operand(h2 q) {
     const h2 q1 = q * splat2((_Float16)kSumScale1);
     const h2 q2 = q * splat2((_Float16)kSumScale2);
-    return h8{q[0], q1[0], q2[0], 0, q[1], q1[1], q2[1], 0};
+    return h8{q[0], q[1], q1[0], q1[1], q2[0], q2[1], 0, 0};
 }
 
 template <int WT>
